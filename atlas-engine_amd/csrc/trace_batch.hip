@@ -123,8 +123,10 @@ __global__ __launch_bounds__(BLOCK) void k_batch_persistent(BatchDev D, const ui
             if (uint32_t(__popcll(__ballot(active))) < threshold) break;
         }
     }
+    // The last wave out resets the counters.  Its atomics need no fence: a
+    // wave's adds to the counters have returned before it adds to ctl[1] (and
+    // a device-scope fence writes back the L2, once per wave).
     if (lane == 0) {
-        __threadfence();
         const uint32_t waves = gridDim.x * (BLOCK / kWave);
         if (atomicAdd(&ctl[1], 1u) == waves - 1) {
             for (uint32_t r = 0; r < kPullRanges; r++) atomicExch(&ctl[kRangeWord * (r + 1)], 0u);

@@ -16,17 +16,22 @@
 // array sized from the tree depth.  Results equal the engine's bit for bit.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "rt_internal.h"
 #include "trace_core.h"
+#include "walk.h"
 
 namespace atlas_rt {
 
 namespace {
 
 constexpr int kWave = 64;
+// 400 - 800 measured the same on 1M - 4M incoherent rays, 200 and 1600 slower.
+constexpr uint32_t kIdleSteps = 400;
 
 template <int BLOCK, int LDS_DEPTH, bool STATS, int NODE_W = 2, bool REG = false, bool FLOAT_SLAB = false>
 __global__ __launch_bounds__(BLOCK) void k_blas_closest(BlasDev B, const float4* __restrict__ rays,
@@ -134,8 +139,10 @@ __global__ __launch_bounds__(BLOCK) void k_blas_closest_persistent(BlasDev B, co
         }
     }
     // Every wave has taken its last ray; the last one out resets the counters.
+    // Its atomics need no fence: a wave's adds to the counters have returned
+    // before it adds to ctl[1] (and a device-scope fence writes back the L2,
+    // once per wave).
     if (lane == 0) {
-        __threadfence();
         const uint32_t waves = gridDim.x * (BLOCK / kWave);
         if (atomicAdd(&ctl[1], 1u) == waves - 1) {
             for (uint32_t r = 0; r < kPullRanges; r++) atomicExch(&ctl[kRangeWord * (r + 1)], 0u);
@@ -144,31 +151,181 @@ __global__ __launch_bounds__(BLOCK) void k_blas_closest_persistent(BlasDev B, co
     }
 }
 
-template <int BLOCK, int LDS_DEPTH>
-__global__ __launch_bounds__(BLOCK) void k_blas_any(BlasDev B, const float4* __restrict__ rays,
-                                                    uint32_t* __restrict__ out, uint32_t count,
-                                                    int32_t* __restrict__ spill, uint32_t cap,
-                                                    uint32_t* __restrict__ ctl) {
-    __shared__ int32_t lds[LDS_DEPTH * BLOCK];
-    const uint32_t gid = blockIdx.x * BLOCK + threadIdx.x;
-    if (gid >= count) return;
-    const float4 r0 = rays[2 * size_t(gid)];
-    const float4 r1 = rays[2 * size_t(gid) + 1];
-    LaneState L;
-    L.slot = -1;
-    if (!any_nan3(r1.x, r1.y, r1.z)) {
-        lane_begin(L, B, r0, r1);
-        const LaneStack<BLOCK, LDS_DEPTH> S{lds, spill, threadIdx.x, gid, gridDim.x * BLOCK};
-        int r;
-        do {
-            r = step_any<BLOCK, LDS_DEPTH>(B, L, S, cap, r1.w);
-        } while (r == kContinue);
-        if (r == kOverflow) {
-            atomicOr(&ctl[2], 1u);
-            L.slot = -1;
+// Words of the flag block that the walk kernels use: the chunk counters of
+// ChunkPull, and whether the launch's rays were found coherent.
+constexpr uint32_t kChunkWord = 8;  // sequence r's at word kRangeWord * (r + 1) + kChunkWord
+constexpr uint32_t kCoherentWord = 3;
+
+// Whether the wave's rays start and run close together: most lanes within a
+// few degrees of the lane beside them, and within a sixteenth of the tree's
+// box.
+__device__ __forceinline__ bool coherent_rays(const BlasDev& B, bool valid, float4 r0, float4 r1) {
+    if (!B.node_count) return true;
+    const float4 a = ldg4(B.nodes), b = ldg4(B.nodes + 1), c = ldg4(B.nodes + 2);
+    const float reach = 0.0625f * fmaxf(fmaxf(fmaxf(a.w, c.y) - fminf(a.x, b.z), fmaxf(b.x, c.z) - fminf(a.y, b.w)),
+                                        fmaxf(b.y, c.w) - fminf(a.z, c.x));
+    const auto beside = [](float v) {
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1 /* quad_perm 1 0 3 2 */, 0xf, 0xf, true));
+    };
+    const float nx = beside(r1.x), ny = beside(r1.y), nz = beside(r1.z);
+    const float dot = r1.x * nx + r1.y * ny + r1.z * nz;
+    const float dd = (r1.x * r1.x + r1.y * r1.y + r1.z * r1.z) * (nx * nx + ny * ny + nz * nz);
+    const float gap = fmaxf(fmaxf(fabsf(r0.x - beside(r0.x)), fabsf(r0.y - beside(r0.y))), fabsf(r0.z - beside(r0.z)));
+    // a NaN direction ends at once: it may run anywhere
+    const bool apart = dot < 0.0f || dot * dot < 0.94f * dd || gap > reach;
+    return uint32_t(__popcll(mask_of(valid && apart))) * 4 < uint32_t(__popcll(mask_of(valid)));
+}
+
+// Before a walk of resident waves: clears their chunk counters and, with
+// `choose`, samples 64 chunks of 64 rays over the batch and notes whether
+// most of them are coherent.
+constexpr uint32_t kBeginBlock = 1024;
+__global__ __launch_bounds__(kBeginBlock) void k_walk_begin(BlasDev B, const float4* __restrict__ rays, uint32_t count,
+                                                            uint32_t* __restrict__ ctl, bool choose) {
+    __shared__ uint32_t coherent;
+    const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    if (tid < kPullRanges) ctl[kRangeWord * (tid + 1) + kChunkWord] = 0;
+    if (!choose) return;
+    if (tid == 0) coherent = 0;
+    __syncthreads();
+    constexpr uint32_t kWaves = kBeginBlock / kWave, kEach = 64 / kWaves;
+    const uint32_t chunks = (count + 63u) / 64u;
+    uint32_t found = 0;
+    for (uint32_t i = 0; i < kEach; i++) {
+        const uint32_t k = uint32_t(uint64_t(wave * kEach + i) * chunks / 64u) * 64u + lane;
+        const bool valid = k < count;
+        float4 r0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), r1 = r0;
+        if (valid) {
+            r0 = rays[2 * size_t(k)];
+            r1 = rays[2 * size_t(k) + 1];
         }
+        found += coherent_rays(B, valid, r0, r1) ? 1u : 0u;
     }
-    out[gid] = L.slot >= 0 ? 1u : 0u;
+    if (lane == 0 && found) atomicAdd(&coherent, found);
+    __syncthreads();
+    if (tid == 0) ctl[kCoherentWord] = coherent * 2 >= 64u ? 1u : 0u;
+}
+
+// Engine-order binary walks (walk.h), by shape:
+//   kOnce   one set of `per_wave` rays per wave;
+//   kPull   resident waves take chunks of 64 rays and refill their idle lanes
+//           from them.
+// chosen: run only if k_walk_begin found the rays coherent (kOnce) or not
+// (kPull); a large batch launches both.  Coherent rays share their nodes'
+// cache lines and end together: a wave per chunk, started in the rays' order
+// by the hardware, loads each node once for many lanes and balances best
+// (1920 x 1080 camera rays over 1.0M triangles: 0.26 ms against 0.39
+// resident).  Incoherent rays end one by one, so lanes are refilled, and their
+// node records go through LDS (NodeStage) while there is work; the last rays,
+// few in each wave, load their nodes directly (1M rays in a random soup of
+// 65,536 triangles: 0.60 ms against 0.84 once).
+//
+// When to refill.  A wave waits until its idle lanes have cost kIdleSteps
+// lane-steps since its last refill, about what a refill costs.  The rays of a
+// refill load beside the hit records of the rays they replace.
+enum class Shape { kOnce, kPull };
+
+template <int BLOCK, int ROWS, bool ANY, Shape SHAPE, int LEAF_DIV>
+__global__ __launch_bounds__(BLOCK, ROWS > 14 ? 3 : 5) void k_blas_walk(BlasDev B, const float4* __restrict__ rays,
+                                                        void* __restrict__ out, int32_t* __restrict__ slots,
+                                                        uint32_t count, int32_t* __restrict__ spill, uint32_t cap,
+                                                        uint32_t* __restrict__ ctl, uint32_t per_wave, bool chosen) {
+    constexpr bool kPulls = SHAPE == Shape::kPull;
+    if (chosen && (ctl[kCoherentWord] != 0) == kPulls) return;
+    __shared__ int32_t lds[ROWS * BLOCK];
+    __shared__ __align__(16) char staged[kPulls ? (BLOCK / kWave) * NodeStage::kBytes : 16];
+    const NodeStage stage(staged);
+    using Stack = WalkStack<BLOCK, ROWS>;
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const Stack S(lds, spill, blockIdx.x * BLOCK + threadIdx.x, gridDim.x * BLOCK, cap);
+    constexpr uint32_t kNone = 0xFFFFFFFFu;
+    Walk w;
+    w.node = kEnd;
+    uint32_t idx = kNone;  // the lane's ray, until its result is written
+    float tmax = 0.0f;
+    ChunkPull pull;
+    uint32_t from = 0, to = 0;   // rays this wave holds and has not started
+    if (kPulls) {
+        pull.init();
+    } else {
+        from = (blockIdx.x * (BLOCK / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave)) * per_wave;
+        to = min(count, from + per_wave);
+    }
+    for (;;) {
+        if (kPulls && from >= to && !pull.dry) {
+            uint32_t chunk;
+            if (pull.take(ctl + kRangeWord + kChunkWord, kRangeWord, (count + 63u) / 64u, chunk)) {
+                from = chunk * 64u;
+                to = from + min(64u, count - from);
+            }
+        }
+        const uint64_t idle = mask_of(w.node == kEnd);
+        const uint32_t k = from + __popcll(idle & ((1ull << lane) - 1));
+        const bool start = w.node == kEnd && k < to;
+        float4 r0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), r1 = r0;
+        if (start) {
+            r0 = rays[2 * size_t(k)];
+            r1 = rays[2 * size_t(k) + 1];
+        }
+        from += uint32_t(__popcll(mask_of(start)));
+        // The results of the rays that ended since the last refill, all at
+        // once: the FP64 refinement runs once per refill round.
+        if (w.node == kEnd && idx != kNone) {
+            if (ANY) {
+                reinterpret_cast<uint32_t*>(out)[idx] = w.slot >= 0 ? 1u : 0u;
+            } else {
+                reinterpret_cast<float4*>(out)[idx] = walk_hit_record(w, B.tris, B.vtx, tmax);
+                if (slots) slots[idx] = w.slot;
+            }
+            idx = kNone;
+        }
+        if (start) {
+            idx = k;
+            tmax = r1.w;
+            walk_begin(w, B.node_count, r0, r1, Stack::bottom(threadIdx.x));
+            if (any_nan3(r1.x, r1.y, r1.z)) w.node = kEnd;
+        }
+        const bool more = from < to || (kPulls && !pull.dry);
+        if (!more && mask_of(idx != kNone) == 0) break;
+        const auto walk = [&](auto through_lds) {
+            uint32_t wasted = 0;
+            uint64_t live = mask_of(w.node != kEnd);
+            while (live != 0 && wasted <= kIdleSteps) {
+                // node steps until enough lanes wait at a leaf
+                uint64_t inner = mask_of(w.node >= 0);
+                while (LEAF_DIV ? uint32_t(__popcll(live ^ inner)) * LEAF_DIV < uint32_t(__popcll(live)) : inner != 0) {
+                    int32_t below = 0;
+                    bool checked = false;
+                    if (through_lds) {
+                        if (w.node >= 0) checked = walk_stack(w, S, below);
+                        stage.fetch(B.nodes, w.node, inner);
+                    }
+                    if (w.node >= 0) {
+                        if (through_lds)
+                            stage.wait();
+                        else
+                            checked = walk_stack(w, S, below);
+                        const NodeRec n = through_lds ? stage.read() : load_node(B.nodes, w.node);
+                        const uint64_t over = walk_node(w, n, checked, below, S, ANY ? ~0ull : 0ull);
+                        if (__builtin_expect(over != 0, 0)) {
+                            atomicOr(&ctl[2], 1u);
+                            if (lane_in(over)) w.slot = -1;
+                        }
+                    }
+                    if (more) wasted += kWave - uint32_t(__popcll(live));
+                    live = mask_of(w.node != kEnd);
+                    inner = mask_of(w.node >= 0);
+                    if (LEAF_DIV == 0 || wasted > kIdleSteps) break;
+                }
+                if (w.node < 0 && w.node != kEnd) walk_leaf(w, B.tris, S, ANY);
+                live = mask_of(w.node != kEnd);
+            }
+        };
+        if (kPulls && more)
+            walk(std::true_type{});
+        else
+            walk(std::false_type{});
+    }
 }
 
 constexpr int kBlock = 128;
@@ -204,6 +361,103 @@ int device_cu_count() {
     return cached;
 }
 
+// Leaf batching: triangle steps once a quarter of a wave's live lanes wait at
+// a leaf.
+constexpr int kLeafDiv = 4;
+
+// The counters and the overflow word, zero between launches.
+static atlas_rt_status ensure_flags(atlas_rt_blas& blas) {
+    if (blas.flags.ptr) return ATLAS_RT_OK;
+    atlas_rt_status st = blas.flags.ensure(kFlagBytes);
+    if (st != ATLAS_RT_OK) return st;
+    ATLAS_HIP_TRY(hipMemset(blas.flags.ptr, 0, kFlagBytes));
+    return ATLAS_RT_OK;
+}
+
+constexpr int kWalkBlock = 256;
+// LDS stack rows: with the staged nodes, five groups of resident waves fit
+// one CU (14 KB + 16.3 KB each).
+constexpr int kWalkRows = 14;
+constexpr uint32_t kWalkGroups = 5;
+
+// Launches below this many rays run once, with as many rays per wave as give
+// every CU eight waves: a wave's step takes as long as its slowest lane's
+// memory access, and all of its lanes' accesses after one another (5,003 rays
+// 0.111 -> 0.093 ms, 16,384 rays 0.194 -> 0.166 ms against 64 per wave).
+constexpr uint32_t kOnceRays = 65536;
+inline uint32_t rays_per_wave(uint32_t count) { return std::min(64u, (count + 2047u) / 2048u); }
+
+// Spill rows of a walk kernel: entries 1 .. cap, of which ROWS - 1 in LDS.
+inline size_t walk_spill_bytes(uint32_t cap, uint32_t rows, size_t threads) {
+    return cap >= rows ? size_t(cap + 1 - rows) * threads * sizeof(int32_t) : 0;
+}
+
+struct WalkArgs {
+    BlasDev B;
+    const float4* rays;
+    void* out;
+    int32_t* slots;
+    uint32_t count;
+    int32_t* spill;
+    uint32_t cap;
+    uint32_t* ctl;
+    hipStream_t stream;
+};
+
+template <bool ANY>
+static void walk_once(const WalkArgs& a, uint32_t groups, uint32_t per_wave, bool chosen) {
+    hipLaunchKernelGGL((k_blas_walk<64, kWalkRows, ANY, Shape::kOnce, 0>), dim3(groups), dim3(64), 0, a.stream, a.B,
+                       a.rays, a.out, a.slots, a.count, a.spill, a.cap, a.ctl, per_wave, chosen);
+}
+
+template <bool ANY, int ROWS = kWalkRows>
+static void walk_pull(const WalkArgs& a, bool leaf_batch, uint32_t groups, bool chosen) {
+    if (leaf_batch)
+        hipLaunchKernelGGL((k_blas_walk<kWalkBlock, ROWS, ANY, Shape::kPull, kLeafDiv>), dim3(groups), dim3(kWalkBlock),
+                           0, a.stream, a.B, a.rays, a.out, a.slots, a.count, a.spill, a.cap, a.ctl, 64u, chosen);
+    else
+        hipLaunchKernelGGL((k_blas_walk<kWalkBlock, ROWS, ANY, Shape::kPull, 0>), dim3(groups), dim3(kWalkBlock), 0,
+                           a.stream, a.B, a.rays, a.out, a.slots, a.count, a.spill, a.cap, a.ctl, 64u, chosen);
+}
+
+static void walk_begin_launch(const WalkArgs& a, bool choose) {
+    hipLaunchKernelGGL(k_walk_begin, dim3(1), dim3(kBeginBlock), 0, a.stream, a.B, a.rays, a.count, a.ctl, choose);
+}
+
+enum class WalkPlan { kAuto, kOnce, kPull, kPullLeafBatch };
+
+template <bool ANY>
+static atlas_rt_status launch_walk(atlas_rt_blas& blas, const TraceLaunch& L, WalkPlan plan) {
+    const bool choose = plan == WalkPlan::kAuto && L.count >= kOnceRays;
+    const bool pull = choose || plan == WalkPlan::kPull || plan == WalkPlan::kPullLeafBatch;
+    const bool once = choose || !pull;
+    const uint32_t per_wave = once && !choose && plan == WalkPlan::kAuto ? rays_per_wave(L.count) : 64u;
+    const uint32_t once_groups = (L.count - 1) / per_wave + 1;
+    const uint32_t pull_groups = uint32_t(device_cu_count()) * kWalkGroups;
+    const uint32_t cap = limit_cap(blas.max_depth + 1, blas.stack_limit);
+    const size_t threads = std::max(once ? size_t(once_groups) * 64 : 0, pull ? size_t(pull_groups) * kWalkBlock : 0);
+    const size_t spill_bytes = walk_spill_bytes(cap, kWalkRows, threads);
+    atlas_rt_status st = ATLAS_RT_OK;
+    if (spill_bytes) st = blas.spill.ensure(spill_bytes);
+    if (st == ATLAS_RT_OK) st = ensure_flags(blas);
+    if (st == ATLAS_RT_OK) st = blas.timing.begin(L.stream);
+    if (st != ATLAS_RT_OK) return st;
+    const WalkArgs a{blas_dev(blas),
+                     reinterpret_cast<const float4*>(L.rays),
+                     L.hits,
+                     L.slots,
+                     L.count,
+                     reinterpret_cast<int32_t*>(blas.spill.ptr),
+                     cap,
+                     reinterpret_cast<uint32_t*>(blas.flags.ptr),
+                     L.stream};
+    if (pull) walk_begin_launch(a, choose);
+    if (once) walk_once<ANY>(a, once_groups, per_wave, choose);
+    if (pull) walk_pull<ANY>(a, plan != WalkPlan::kPull, pull_groups, choose);
+    ATLAS_HIP_TRY(hipGetLastError());
+    return blas.timing.end(L.stream);
+}
+
 static atlas_rt_status prepare(atlas_rt_blas& blas, uint32_t threads, uint32_t lds_depth, uint32_t& cap,
                                int node_w = 2) {
     // The binary stack never holds more entries than the deepest leaf's
@@ -214,12 +468,7 @@ static atlas_rt_status prepare(atlas_rt_blas& blas, uint32_t threads, uint32_t l
         atlas_rt_status st = blas.spill.ensure(need);
         if (st != ATLAS_RT_OK) return st;
     }
-    if (!blas.flags.ptr) {
-        atlas_rt_status st = blas.flags.ensure(kFlagBytes);
-        if (st != ATLAS_RT_OK) return st;
-        ATLAS_HIP_TRY(hipMemset(blas.flags.ptr, 0, kFlagBytes));
-    }
-    return ATLAS_RT_OK;
+    return ensure_flags(blas);
 }
 
 template <int NODE_W, bool REG, bool FLOAT_SLAB = false, int LEAF_DIV = 0>
@@ -231,21 +480,8 @@ static void launch_persistent(const BlasDev& B, const TraceLaunch& L, uint32_t g
                        L.slots, L.count, spill, cap, ctl, L.refill ? L.refill : 40u);
 }
 
-// Leaf batching: triangle steps once a quarter of a wave's live lanes wait at
-// a leaf.
-constexpr int kLeafDiv = 4;
-
-// ATLAS_RT_KERNEL_AUTO: resident leaf-batched waves (the fastest
-// engine-exact variant on C0) for large batches, one ray per lane for small
-// ones, where a resident grid would mostly idle.
-constexpr uint32_t kAutoPersistentRays = 65536;
-
-atlas_rt_status launch_blas_closest(atlas_rt_blas& blas, const TraceLaunch& L0) {
-    if (L0.count == 0) return ATLAS_RT_OK;
-    TraceLaunch L = L0;
-    if (L.kernel == ATLAS_RT_KERNEL_AUTO && !L.visits)
-        L.kernel = L.count >= kAutoPersistentRays ? (ATLAS_RT_KERNEL_BVH2_PERSISTENT | ATLAS_RT_KERNEL_LEAF_BATCH)
-                                                  : ATLAS_RT_KERNEL_BVH2_EXACT;
+atlas_rt_status launch_blas_closest(atlas_rt_blas& blas, const TraceLaunch& L) {
+    if (L.count == 0) return ATLAS_RT_OK;
     const BlasDev B = blas_dev(blas);
     uint32_t* ctl = reinterpret_cast<uint32_t*>(blas.flags.ptr);
     const int base = L.kernel & ATLAS_RT_KERNEL_VARIANT_MASK;
@@ -253,18 +489,19 @@ atlas_rt_status launch_blas_closest(atlas_rt_blas& blas, const TraceLaunch& L0) 
     const bool fslab = (L.kernel & ATLAS_RT_KERNEL_SLAB_FLOAT) != 0;
     const bool leaf_batch = (L.kernel & ATLAS_RT_KERNEL_LEAF_BATCH) != 0;
     const bool persistent = !L.visits && base >= ATLAS_RT_KERNEL_BVH2_PERSISTENT;
+    if (!L.visits && !reg && !fslab && base <= ATLAS_RT_KERNEL_BVH2_PERSISTENT)
+        return launch_walk<false>(blas, L,
+                                  base == ATLAS_RT_KERNEL_AUTO ? WalkPlan::kAuto
+                                  : !persistent                ? WalkPlan::kOnce
+                                  : leaf_batch                 ? WalkPlan::kPullLeafBatch
+                                                               : WalkPlan::kPull);
     const int node_w = base == ATLAS_RT_KERNEL_BVH4 ? 4 : (base == ATLAS_RT_KERNEL_BVH8 ? 8 : 2);
     atlas_rt_status st;
     uint32_t cap = 0;
     if (persistent) {
-        // Resident grid: 256-lane groups per CU.  Four in general (measured
-        // on C0: 0.98 ms against 1.06 ms with eight; fewer resident waves
-        // keep more of the tree in each XCD's L2); five for the binary exact
-        // leaf-batched kernel, whose 96 VGPRs leave room for a fifth wave per
-        // SIMD (C0: 0.824 against 0.852 ms, where the float-slab variants
-        // slow down with five; six, built for 80 VGPRs, took 0.84 ms).
-        const bool five = node_w == 2 && leaf_batch && !reg && !fslab;
-        const uint32_t groups = uint32_t(device_cu_count()) * (five ? 5u : 4u);
+        // Resident grid: four 256-lane groups per CU (fewer resident waves
+        // keep more of the tree in each XCD's L2).
+        const uint32_t groups = uint32_t(device_cu_count()) * 4u;
         st = prepare(blas, groups * kPBlock, kPLdsDepth, cap, node_w);
         if (st != ATLAS_RT_OK) return st;
         ctl = reinterpret_cast<uint32_t*>(blas.flags.ptr);
@@ -276,14 +513,12 @@ atlas_rt_status launch_blas_closest(atlas_rt_blas& blas, const TraceLaunch& L0) 
                 reg ? launch_persistent<2, true, true, kLeafDiv>(B, L, groups, spill, cap, ctl)
                     : launch_persistent<2, false, true, kLeafDiv>(B, L, groups, spill, cap, ctl);
             else
-                reg ? launch_persistent<2, true, false, kLeafDiv>(B, L, groups, spill, cap, ctl)
-                    : launch_persistent<2, false, false, kLeafDiv>(B, L, groups, spill, cap, ctl);
+                launch_persistent<2, true, false, kLeafDiv>(B, L, groups, spill, cap, ctl);
         } else if (node_w == 2 && fslab)
             reg ? launch_persistent<2, true, true>(B, L, groups, spill, cap, ctl)
                 : launch_persistent<2, false, true>(B, L, groups, spill, cap, ctl);
         else if (node_w == 2)
-            reg ? launch_persistent<2, true>(B, L, groups, spill, cap, ctl)
-                : launch_persistent<2, false>(B, L, groups, spill, cap, ctl);
+            launch_persistent<2, true>(B, L, groups, spill, cap, ctl);
         else if (node_w == 4 && leaf_batch && fslab)
             reg ? launch_persistent<4, true, true, kLeafDiv>(B, L, groups, spill, cap, ctl)
                 : launch_persistent<4, false, true, kLeafDiv>(B, L, groups, spill, cap, ctl);
@@ -325,15 +560,10 @@ atlas_rt_status launch_blas_closest(atlas_rt_blas& blas, const TraceLaunch& L0) 
         ctl = reinterpret_cast<uint32_t*>(blas.flags.ptr);
         st = blas.timing.begin(L.stream);
         if (st != ATLAS_RT_OK) return st;
-        if (L.visits)
-            hipLaunchKernelGGL((k_blas_closest<kBlock, kLdsDepth, true>), dim3(grid), dim3(kBlock), 0, L.stream, B,
-                               reinterpret_cast<const float4*>(L.rays), reinterpret_cast<float4*>(L.hits), L.slots,
-                               reinterpret_cast<uint2*>(L.visits), L.count,
-                               reinterpret_cast<int32_t*>(blas.spill.ptr), cap, ctl);
-        else
-            hipLaunchKernelGGL((k_blas_closest<kBlock, kLdsDepth, false>), dim3(grid), dim3(kBlock), 0, L.stream, B,
-                               reinterpret_cast<const float4*>(L.rays), reinterpret_cast<float4*>(L.hits), L.slots,
-                               nullptr, L.count, reinterpret_cast<int32_t*>(blas.spill.ptr), cap, ctl);
+        hipLaunchKernelGGL((k_blas_closest<kBlock, kLdsDepth, true>), dim3(grid), dim3(kBlock), 0, L.stream, B,
+                           reinterpret_cast<const float4*>(L.rays), reinterpret_cast<float4*>(L.hits), L.slots,
+                           reinterpret_cast<uint2*>(L.visits), L.count, reinterpret_cast<int32_t*>(blas.spill.ptr),
+                           cap, ctl);
     }
     ATLAS_HIP_TRY(hipGetLastError());
     return blas.timing.end(L.stream);
@@ -404,25 +634,31 @@ atlas_rt_status launch_blas_closest_noalloc(const atlas_rt_blas& blas, const Tra
                                                    " (use atlas_rt_trace_closest_rays)");
     uint32_t* ctl = reinterpret_cast<uint32_t*>(sp);
     int32_t* spill = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(sp) + kNoAllocCtlBytes);
-    // the range counters, the wave counter and the overflow flag start at zero
+    // the counters and the overflow flag start at zero
     hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(256), 0, L.stream, ctl, uint32_t(kNoAllocCtlBytes / 4));
     const BlasDev B = blas_dev(blas);
     const bool reg = (L.kernel & ATLAS_RT_KERNEL_STACK_REGISTER) != 0;
     const bool fslab = (L.kernel & ATLAS_RT_KERNEL_SLAB_FLOAT) != 0;
     const bool leaf_batch = (L.kernel & ATLAS_RT_KERNEL_LEAF_BATCH) != 0;
-    if (leaf_batch) {
+    if (!reg && !fslab) {
+        // 24 stack rows leave room for three groups per CU; their spill rows
+        // (one more than the persistent kernels' above) fit the scratch
+        const WalkArgs a{B,      reinterpret_cast<const float4*>(L.rays), L.hits, L.slots, L.count,
+                         spill,  cap,                                    ctl,    L.stream};
+        static_assert(kPLdsDepth == 24, "the refusal above is the spill bound");
+        const uint32_t walk_groups = uint32_t(device_cu_count()) * 3;
+        walk_pull<false, kPLdsDepth>(a, leaf_batch, walk_groups, false);
+    } else if (leaf_batch) {
         if (fslab)
             reg ? launch_persistent<2, true, true, kLeafDiv>(B, L, groups, spill, cap, ctl)
                 : launch_persistent<2, false, true, kLeafDiv>(B, L, groups, spill, cap, ctl);
         else
-            reg ? launch_persistent<2, true, false, kLeafDiv>(B, L, groups, spill, cap, ctl)
-                : launch_persistent<2, false, false, kLeafDiv>(B, L, groups, spill, cap, ctl);
+            launch_persistent<2, true, false, kLeafDiv>(B, L, groups, spill, cap, ctl);
     } else if (fslab) {
         reg ? launch_persistent<2, true, true>(B, L, groups, spill, cap, ctl)
             : launch_persistent<2, false, true>(B, L, groups, spill, cap, ctl);
     } else {
-        reg ? launch_persistent<2, true>(B, L, groups, spill, cap, ctl)
-            : launch_persistent<2, false>(B, L, groups, spill, cap, ctl);
+        launch_persistent<2, true>(B, L, groups, spill, cap, ctl);
     }
     ATLAS_HIP_TRY(hipGetLastError());
     return ATLAS_RT_OK;
@@ -430,17 +666,7 @@ atlas_rt_status launch_blas_closest_noalloc(const atlas_rt_blas& blas, const Tra
 
 atlas_rt_status launch_blas_any(atlas_rt_blas& blas, const TraceLaunch& L) {
     if (L.count == 0) return ATLAS_RT_OK;
-    const uint32_t grid = (L.count + kBlock - 1) / kBlock;
-    uint32_t cap = 0;
-    atlas_rt_status st = prepare(blas, grid * kBlock, kLdsDepth, cap);
-    if (st != ATLAS_RT_OK) return st;
-    st = blas.timing.begin(L.stream);
-    if (st != ATLAS_RT_OK) return st;
-    hipLaunchKernelGGL((k_blas_any<kBlock, kLdsDepth>), dim3(grid), dim3(kBlock), 0, L.stream, blas_dev(blas),
-                       reinterpret_cast<const float4*>(L.rays), reinterpret_cast<uint32_t*>(L.hits), L.count,
-                       reinterpret_cast<int32_t*>(blas.spill.ptr), cap, reinterpret_cast<uint32_t*>(blas.flags.ptr));
-    ATLAS_HIP_TRY(hipGetLastError());
-    return blas.timing.end(L.stream);
+    return launch_walk<true>(blas, L, WalkPlan::kAuto);
 }
 
 }  // namespace atlas_rt

@@ -34,6 +34,31 @@ __device__ __forceinline__ uint32_t xcc_id() {
     return v & 0xfu;
 }
 
+// The sequence a wave turns to when its own, `cur`, has run dry: the next one
+// after it, cyclically, whose counter has not reached its length; kPullRanges
+// when there is none.  Lane r passes sequence r's length; the whole wave is
+// active.  One load reads all the counters, where an atomic add per dry
+// sequence has every wave of the chip add to the same eight words as a launch
+// ends.
+__device__ __forceinline__ uint32_t next_sequence(const uint32_t* counters, uint32_t stride, uint32_t length,
+                                                  uint32_t cur) {
+    const uint32_t lane = threadIdx.x & 63u;
+    bool left = false;
+    if (lane < kPullRanges)
+        left = __hip_atomic_load(&counters[size_t(lane) * stride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < length;
+    const uint32_t m = uint32_t(__builtin_amdgcn_ballot_w64(left));
+    if (m == 0) return kPullRanges;
+    const uint32_t after = (m | m << kPullRanges) >> (cur + 1);
+    return (cur + 1 + uint32_t(__builtin_ctz(after))) % kPullRanges;
+}
+
+// The first active lane's atomic add, for the whole wave.
+__device__ __forceinline__ uint32_t wave_add(uint32_t* counter, uint32_t n) {
+    uint32_t j = 0;
+    if (__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) == 0) j = atomicAdd(counter, n);
+    return __builtin_amdgcn_readfirstlane(j);
+}
+
 // A wave's position in the kPullRanges ranges of [0, total): counter r sits
 // at counters[r * stride] (32-bit words).  take() is called by one lane: it
 // reserves n items from the current range, moving to the next range while
@@ -65,6 +90,40 @@ struct RangePull {
     __device__ __forceinline__ void broadcast(int from) {
         cur = __shfl(cur, from, 64);
         dry = __shfl(dry, from, 64);
+    }
+};
+
+// A wave's position in the kPullRanges interleaved sequences of the chunks of
+// 64 items of [0, total): sequence r holds chunks r, r + kPullRanges, ...,
+// its counter at counters[r * stride].  Items start in about their own order
+// over the whole chip (camera rays: the expensive rows of an image are not
+// left to one XCD's waves, nor to the end), from one counter per XCD.
+struct ChunkPull {
+    uint32_t cur;
+    bool dry;
+    __device__ __forceinline__ void init() {
+        cur = xcc_id() % kPullRanges;
+        dry = false;
+    }
+    // The next chunk of the wave's sequence, all of the wave active; turns to
+    // another when it is dry, false once all are.
+    __device__ __forceinline__ bool take(uint32_t* counters, uint32_t stride, uint32_t chunks, uint32_t& chunk) {
+        while (!dry) {
+            const uint32_t n = length(chunks, cur);
+            if (n) {
+                const uint32_t j = wave_add(&counters[size_t(cur) * stride], 1u);
+                if (j < n) {
+                    chunk = j * kPullRanges + cur;
+                    return true;
+                }
+            }
+            cur = next_sequence(counters, stride, length(chunks, min(threadIdx.x & 63u, kPullRanges - 1u)), cur);
+            dry = cur == kPullRanges;
+        }
+        return false;
+    }
+    static __device__ __forceinline__ uint32_t length(uint32_t chunks, uint32_t r) {
+        return r < chunks ? (chunks - r + kPullRanges - 1u) / kPullRanges : 0u;
     }
 };
 

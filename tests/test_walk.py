@@ -1,0 +1,125 @@
+"""The engine-exact walk (csrc/walk.h) decides boxes from float products with a margin and settles near ties in
+further stages; its hits must stay the oracle's bit for bit where those ties are common: flat boxes, planes shared by
+both children, rays along axes and through edges, distances equal to the current hit, tmin in and on boxes, directions
+outside the margin's premises, stacks deeper than the LDS rows; and over the launch shapes' edges (rays per wave,
+chunks of 64, coherent or incoherent batches)."""
+import numpy as np
+import pytest
+
+import atlas_rt
+import oracle_rt
+import rt_cases
+from atlas_rt import _abi
+from atlas_rt import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def boxes_mesh(g, n=700):
+    """Axis-aligned boxes on a coarse lattice: flat triangles' boxes, many shared and coincident planes."""
+    lo = g.integers(-10, 10, (n, 3)).astype(np.float64) * 0.5
+    hi = lo + g.integers(1, 4, (n, 3)) * 0.5
+    tris = []
+    for a, b in zip(lo, hi):
+        p = [np.array([(a, b)[i & 1][0], (a, b)[(i >> 1) & 1][1], (a, b)[i >> 2][2]]) for i in range(8)]
+        for q in ((0, 1, 3, 2), (4, 5, 7, 6), (0, 1, 5, 4), (2, 3, 7, 6), (0, 2, 6, 4), (1, 3, 7, 5)):
+            tris.append(np.concatenate([p[q[0]], p[q[1]], p[q[2]]]))
+            tris.append(np.concatenate([p[q[0]], p[q[2]], p[q[3]]]))
+    return np.asarray(tris, np.float32)
+
+
+def strip_mesh(n=3000):
+    """Triangles of growing size along x: a tree as deep as the builder makes it."""
+    x = np.cumsum(1.02 ** np.arange(n) * 1e-3)
+    t = np.zeros((n, 9))
+    t[:, 0], t[:, 3], t[:, 6] = x, x * 1.01, x
+    t[:, 4], t[:, 8] = x * 0.02, x * 0.02
+    return t.astype(np.float32)
+
+
+def meshes(g):
+    return {"soup": W.triangle_soup(3000, g), "boxes": boxes_mesh(g), "height": W.heightfield(64), "strip": strip_mesh(),
+            "one": W.triangle_soup(1, g), "two": W.triangle_soup(2, g)}
+
+
+def hard_rays(g, verts, n):
+    """Rays at the decisions' edges, an eighth of each kind."""
+    rays = W.random_rays(n, g)
+    v = verts.reshape(-1, 3).astype(np.float64)
+    lo, hi = v.min(axis=0), v.max(axis=0)
+    size = np.maximum(hi - lo, 1e-3)
+    o = lo - 0.2 * size + g.uniform(0, 1.4, (n, 3)) * size
+    target = v[g.integers(0, len(v), n)]
+    d = target - o
+    kind = np.arange(n) % 8
+    o[kind == 1] = target[kind == 1]                                     # from a vertex
+    d[kind == 1] = g.standard_normal((np.count_nonzero(kind == 1), 3))
+    axis = g.integers(0, 3, n)
+    along = np.eye(3)[axis] * g.choice([-1.0, 1.0], n)[:, None]
+    k = kind == 2                                                         # along an axis, towards a vertex's line
+    d[k] = along[k]
+    o[k] = target[k] - along[k] * size.max() * g.uniform(0, 2, k.sum())[:, None]
+    k = kind == 3                                                         # in a lattice plane: a zero component
+    d[k] = d[k] * (1 - np.abs(along[k]))
+    o[k] = np.round(o[k] * 2) / 2
+    k = kind == 4                                                         # steep: subnormal and tiny components
+    d[k] = d[k] * np.where(np.abs(along[k]) > 0, g.choice([1e-45, 1e-39, 1e-30, 1e-8], k.sum())[:, None], 1.0)
+    k = kind == 5                                                         # long and short directions
+    d[k] = d[k] * g.choice([1e-30, 1e-10, 1e10, 1e38], k.sum())[:, None]
+    rays["origin"] = o.astype(np.float32)
+    with np.errstate(over="ignore"):
+        rays["direction"] = d.astype(np.float32)
+    rays["tmin"] = g.choice(np.array([0.0, 1e-4, 1.0, -1.0], np.float32), n)
+    rays["tmax"] = g.choice(np.array([1e12, np.inf, 2.0, 0.0], np.float32), n)
+    k = kind == 6                                                         # tmax, then tmin, on the vertex itself
+    rays["direction"][k] = (target[k] - o[k]).astype(np.float32)
+    rays["tmax"][k] = 1.0
+    k = kind == 7
+    rays["tmin"][k] = 1.0
+    return rays
+
+
+def trace(torch, blas, rays, kernel):
+    d = torch.from_numpy(rays.view(np.float32).reshape(-1, 8).copy()).cuda()
+    h = torch.full((len(rays), 4), -7.0, device="cuda")
+    s = torch.full((len(rays),), -7, dtype=torch.int32, device="cuda")
+    blas.trace_closest(d, h, s, kernel=kernel)
+    a = torch.full((len(rays),), -7, dtype=torch.int32, device="cuda")
+    blas.trace_any(d, a)
+    torch.cuda.synchronize()
+    return h.cpu().numpy().view(atlas_rt.HIT_DTYPE).reshape(-1), s.cpu().numpy(), a.cpu().numpy().astype(np.uint32)
+
+
+@pytest.mark.parametrize("name", ["soup", "boxes", "height", "strip", "one", "two"])
+def test_hard_rays_bit_exact(torch_cuda, name):
+    g = W.rng(5, 1)
+    verts = meshes(g)[name]
+    blas = atlas_rt.Blas.build(verts)
+    nodes, tris, orig = blas.export()
+    rays = hard_rays(g, verts, 70001)
+    ref, slots = oracle_rt.trace_closest(nodes, tris, orig, rays)
+    any_ref = oracle_rt.trace_any(nodes, tris, rays)
+    for kernel in (0, 1, 2, 2 | _abi.KERNEL_LEAF_BATCH):
+        h, s, a = trace(torch_cuda, blas, rays, kernel)
+        bad = np.nonzero(np.any(rt_cases.hit_bits(h) != rt_cases.hit_bits(ref), axis=1) | (s != slots))[0]
+        assert len(bad) == 0, f"{name} kernel {kernel}: {len(bad)} rays, first {bad[:4]} {rays[bad[:2]]} {h[bad[:2]]} {ref[bad[:2]]}"
+    bad = np.nonzero(a != any_ref)[0]
+    assert len(bad) == 0, f"{name} any: {len(bad)} rays, first {bad[:4]} {rays[bad[:2]]}"
+
+
+@pytest.mark.parametrize("count", [1, 2, 63, 64, 65, 2048, 2049, 5003, 65535, 65536, 65537, 131073])
+@pytest.mark.parametrize("coherent", [False, True])
+def test_launch_shapes_bit_exact(torch_cuda, count, coherent):
+    g = W.rng(5, 2)
+    verts = W.heightfield(64)
+    blas = atlas_rt.Blas.build(verts)
+    nodes, tris, orig = blas.export()
+    if coherent:
+        rays = W.pinhole_rays(512, 257, (31.0, 60.0, -9.0), 0.0, 30.0)[:count]
+    else:
+        rays = W.random_rays(count, g, extent=40.0)
+    rays["direction"][::97] = np.nan
+    ref, slots = oracle_rt.trace_closest(nodes, tris, orig, rays)
+    h, s, a = trace(torch_cuda, blas, rays, 0)
+    assert np.array_equal(rt_cases.hit_bits(h), rt_cases.hit_bits(ref)) and np.array_equal(s, slots)
+    assert np.array_equal(a, oracle_rt.trace_any(nodes, tris, rays))
