@@ -39,8 +39,22 @@
 #include <stdint.h>
 
 #include "rt_device.h"
+#include "rt_internal.h"
 
 namespace atlas_rt {
+
+// What a walk needs of a BLAS record, read from a table in global memory.
+struct BlasView {
+    const float4* nodes;
+    const float4* tris;
+    const float4* vtx;
+    uint32_t node_count;
+};
+
+__device__ __forceinline__ BlasView blas_view(const BlasDev* p) {
+    const __attribute__((address_space(1))) BlasDev* g = (const __attribute__((address_space(1))) BlasDev*)p;
+    return BlasView{g->nodes, g->tris, g->vtx, g->node_count};
+}
 
 constexpr int32_t kEnd = INT32_MIN;   // node of a lane whose walk has ended
 
