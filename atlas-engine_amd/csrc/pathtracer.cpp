@@ -270,9 +270,9 @@ size_t atlas_rt::pt::slot_spill_bytes(uint32_t rays, uint32_t cap) {
         const size_t grid_threads = (size_t(rays) + kGridBlock - 1) / kGridBlock * kGridBlock;
         need = size_t(cap - kGridLds) * grid_threads * sizeof(int32_t);
     }
-    if (cap > uint32_t(kResidentLds)) {
+    if (cap >= uint32_t(kResidentLds)) {  // the walk's rows 1 .. cap (row 0 is padding)
         const size_t lanes = size_t(device_cu_count()) * kResidentGroupsPerCu * kResidentBlock;
-        need = std::max(need, size_t(cap - kResidentLds) * lanes * sizeof(int32_t));
+        need = std::max(need, size_t(cap + 1 - kResidentLds) * lanes * sizeof(int32_t));
     }
     return need;
 }

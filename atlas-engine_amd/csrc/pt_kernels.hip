@@ -29,6 +29,7 @@
 #include "pathtracer.h"
 #include "pt_device.h"
 #include "trace_world_core.h"
+#include "world_walk.h"
 
 namespace atlas_rt {
 namespace pt {
@@ -921,6 +922,8 @@ __global__ __launch_bounds__(kFrameBlock, OCC) void k_frame_persistent(ShadeArgs
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const LaneStack<kFrameBlock, kFrameLds> S{lds, spill, tid, blockIdx.x * kFrameBlock + tid,
                                               gridDim.x * kFrameBlock};
+    using Stack = WalkStack<kFrameBlock, kFrameLds>;
+    const Stack SW(lds, spill, blockIdx.x * kFrameBlock + tid, gridDim.x * kFrameBlock, cap);
     FrameCtl* const ctl0 = A.ctl;  // frame f's seeds and counts in ctl0[f]; ctl0[0].pull counts paths
     const WorldDev W = A.world;
     const AlphaArgs& AA = A.alpha;
@@ -932,8 +935,16 @@ __global__ __launch_bounds__(kFrameBlock, OCC) void k_frame_persistent(ShadeArgs
     const V btm = mk(G.cam.bottom[0], G.cam.bottom[1], G.cam.bottom[2]);
     const V loc = mk(G.cam.loc[0], G.cam.loc[1], G.cam.loc[2]);
 
-    WorldLane L;
-    world_begin(L, make_float4(0.0f, 0.0f, 0.0f, 0.0f), make_float4(1.0f, 0.0f, 0.0f, 0.0f));
+    WorldLane L;  // the lane's walk over worlds with opacity
+    WorldWalk K;  // over opaque ones
+    const auto begin = [&](float4 r0, float4 r1) {
+        if (ALPHA)
+            world_begin(L, r0, r1);
+        else
+            world_walk_begin(K, W, r0, r1, Stack::bottom(tid));
+    };
+    begin(make_float4(0.0f, 0.0f, 0.0f, 0.0f), make_float4(1.0f, 0.0f, 0.0f, 0.0f));
+    K.w.node = kEnd;
     int phase = 0;       // 0 idle, 1 closest hit, 2 shadow ray
     bool ready = false;  // the walk of this phase has ended (result in L / rstat)
     int rstat = kDone;
@@ -1010,9 +1021,9 @@ __global__ __launch_bounds__(kFrameBlock, OCC) void k_frame_persistent(ShadeArgs
                             p2 = make_float4(1.0f, 1.0f, 1.0f, 0.0f);
                             bounce = 0;
                             phase = 1;
-                            world_begin(L, make_float4(p0.x, p0.y, p0.z, 0.0f),
-                                        make_float4(p1.x, p1.y, p1.z, kInf));
+                            begin(make_float4(p0.x, p0.y, p0.z, 0.0f), make_float4(p1.x, p1.y, p1.z, kInf));
                             ready = any_nan3(p1.x, p1.y, p1.z);
+                            if (ready) K.w.node = kEnd;
                             rstat = kDone;
                             if (STATS) c_closest++;
                         }
@@ -1025,32 +1036,34 @@ __global__ __launch_bounds__(kFrameBlock, OCC) void k_frame_persistent(ShadeArgs
             continue;
         }
         // walk until enough lanes have ended their walk
-        for (;;) {
+        if (!ALPHA) {
+            const auto count = [&] {
+                struct Counts {
+                    uint32_t &n, &t, &i;
+                    __device__ __forceinline__ void node() { n++; }
+                    __device__ __forceinline__ void triangle() { t++; }
+                    __device__ __forceinline__ void instance() { i++; }
+                };
+                if constexpr (STATS)
+                    return Counts{c_nodes, c_tris, c_insts};
+                else
+                    return NoCount{};
+            };
+            auto counts = count();
+            const uint64_t over = world_walk<true>(K, W, SW, mask_of(phase == 2),
+                                                   phase == 1 ? ATLAS_RT_MASK_ALL : ATLAS_RT_MASK_SHADOW, counts);
+            ready = phase != 0;
+            rstat = lane_in(over) ? kOverflow : kDone;
+        }
+        for (; ALPHA;) {
             if (phase != 0 && !ready) {
                 int r;
-                if (ALPHA) {
-                    if (phase == 1) {
-                        const AcceptOpaque acc{TriOpacity{W, AA}};
-                        r = world_step_closest<kFrameBlock, kFrameLds>(L, W, ATLAS_RT_MASK_ALL, S, cap, acc);
-                    } else {
-                        const TriOpacity op{W, AA};
-                        r = world_step_transparency<kFrameBlock, kFrameLds>(L, W, ATLAS_RT_MASK_SHADOW, L.hitT, S,
-                                                                            cap, op);
-                    }
+                if (phase == 1) {
+                    const AcceptOpaque acc{TriOpacity{W, AA}};
+                    r = world_step_closest<kFrameBlock, kFrameLds>(L, W, ATLAS_RT_MASK_ALL, S, cap, acc);
                 } else {
-                    if (STATS) {
-                        // the step's kind, as world_step_mixed decides it
-                        const bool top = L.sp + 1 < L.tlas_index;
-                        if (top && L.node < 0)
-                            c_insts++;
-                        else if (top || L.node >= 0)
-                            c_nodes++;
-                        else
-                            c_tris++;
-                    }
-                    r = world_step_mixed<kFrameBlock, kFrameLds>(L, W, phase == 1 ? ATLAS_RT_MASK_ALL
-                                                                                   : ATLAS_RT_MASK_SHADOW,
-                                                                 phase == 2, S, cap);
+                    const TriOpacity op{W, AA};
+                    r = world_step_transparency<kFrameBlock, kFrameLds>(L, W, ATLAS_RT_MASK_SHADOW, L.hitT, S, cap, op);
                 }
                 if (r != kContinue) {
                     ready = true;
@@ -1067,9 +1080,9 @@ __global__ __launch_bounds__(kFrameBlock, OCC) void k_frame_persistent(ShadeArgs
             int32_t slot = -1, inst = -1;
             if (rstat == kOverflow)
                 atomicOr(&flags[2], 1u);
-            else if (L.slot >= 0) {
-                slot = L.slot;
-                inst = L.inst;
+            else if ((ALPHA ? L.slot : K.w.slot) >= 0) {
+                slot = ALPHA ? L.slot : K.w.slot;
+                inst = ALPHA ? L.inst : K.inst;
             }
             if (STATS) c_hits += slot >= 0;
             if (bounce == 0 && G.hit0) {
@@ -1077,7 +1090,8 @@ __global__ __launch_bounds__(kFrameBlock, OCC) void k_frame_persistent(ShadeArgs
                 G.hit0[G.spf ? id / G.spf : id] = slot >= 0 ? 1 : 0;
             }
             ShadeOut so;
-            shade_path(A, ctl, Lpix, bounce, p0, p1, p2, make_int4(__float_as_int(L.hitT), slot, inst, 0), so);
+            shade_path(A, ctl, Lpix, bounce, p0, p1, p2, make_int4(__float_as_int(ALPHA ? L.hitT : K.w.t), slot, inst, 0),
+                       so);
             if (CACHE) {
                 // the path ends with a cache query: one counter update per wave
                 const uint64_t qm = __ballot(so.query);
@@ -1103,8 +1117,8 @@ __global__ __launch_bounds__(kFrameBlock, OCC) void k_frame_persistent(ShadeArgs
             }
             if (so.shadow) {
                 shc = so.sh[2];
-                world_begin(L, make_float4(so.sh[0].x, so.sh[0].y, so.sh[0].z, 0.0f),
-                            make_float4(so.sh[1].x, so.sh[1].y, so.sh[1].z, so.sh[1].w));
+                begin(make_float4(so.sh[0].x, so.sh[0].y, so.sh[0].z, 0.0f),
+                      make_float4(so.sh[1].x, so.sh[1].y, so.sh[1].z, so.sh[1].w));
                 phase = 2;
                 ready = false;
                 if (STATS) c_shadow++;
@@ -1115,7 +1129,7 @@ __global__ __launch_bounds__(kFrameBlock, OCC) void k_frame_persistent(ShadeArgs
             if (rstat == kOverflow) {
                 atomicOr(&flags[2], 1u);
             } else {
-                const float vis = ALPHA ? L.trans : (L.slot >= 0 ? 0.0f : 1.0f);
+                const float vis = ALPHA ? L.trans : (K.w.slot >= 0 ? 0.0f : 1.0f);
                 if (vis != 0.0f) {
                     V cc = mk(shc.x, shc.y, shc.z) * vis;
                     if (bounce > 0) {
@@ -1142,9 +1156,10 @@ __global__ __launch_bounds__(kFrameBlock, OCC) void k_frame_persistent(ShadeArgs
         }
         if (pending) {
             bounce++;
-            world_begin(L, make_float4(p0.x, p0.y, p0.z, 0.0f), make_float4(p1.x, p1.y, p1.z, kInf));
+            begin(make_float4(p0.x, p0.y, p0.z, 0.0f), make_float4(p1.x, p1.y, p1.z, kInf));
             phase = 1;
             ready = any_nan3(p1.x, p1.y, p1.z);
+            if (ready) K.w.node = kEnd;
             rstat = kDone;
             if (STATS) c_closest++;
         } else {
