@@ -127,27 +127,41 @@ __device__ __forceinline__ void lane_features(const NrcDev& P, const float4* __r
     }
 }
 
-// Scatter d(loss)/d(feature) of the lane's hash features into the FP32
-// table gradient.
-__device__ __forceinline__ void lane_table_grad(const NrcDev& P, const float4* __restrict__ q, uint32_t qi, int g,
-                                                const float (&df)[8], float* __restrict__ grad) {
-    const float4 a = q[3 * (size_t)qi];
-    const float x = clamp01((a.x - P.bmin[0]) * P.binv[0]);
-    const float y = clamp01((a.y - P.bmin[1]) * P.binv[1]);
-    const float z = clamp01((a.z - P.bmin[2]) * P.binv[2]);
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int lev = slot_level(g, j);
-        if (lev < 0 || lev >= (int)P.levels) continue;
-        const float d0 = df[2 * j], d1 = df[2 * j + 1];
-        if (d0 == 0.0f && d1 == 0.0f) continue;
-        uint32_t idx[8];
-        float w[8];
-        level_corners(P, lev, x, y, z, idx, w);
-#pragma unroll
-        for (int cc = 0; cc < 8; cc++) {
-            atomicAdd(grad + 2 * (size_t)idx[cc], w[cc] * d0);
-            atomicAdd(grad + 2 * (size_t)idx[cc] + 1, w[cc] * d1);
+// Scatter d(loss)/d(feature) of a wave's 32 queries into the FP32 table
+// gradient.  The atomics are bound by the memory requests they make, about 20
+// a nanosecond over the chip wherever they go, not by their number: one lane
+// per feature with its corners in turn makes one request per atomic.  Here 16
+// lanes take the 8 corners and both features of one query's cell, the two
+// corners along x and their features in four adjacent lanes: 16 adjacent
+// bytes at a dense level, mostly one cache line at a hashed one (x enters the
+// hash unmultiplied), so a request carries about four atomics.
+//   df:  [32 queries][kDfStride] feature gradients, level-major pairs
+//   pos: [32 queries][3] positions in [0, 1]
+constexpr int kDfStride = 25;
+__device__ __forceinline__ void wave_table_grad(const NrcDev& P, const float* df, const float* pos, uint32_t queries,
+                                                int lane, float* __restrict__ grad) {
+    const int f = lane & 1, cx = (lane >> 1) & 1, cy = (lane >> 2) & 1, cz = (lane >> 3) & 1;
+    const uint32_t T = 1u << P.log2_t;
+    for (uint32_t lev = 0; lev < P.levels; lev++) {
+        const float R = P.res[lev];
+        const bool dense = (P.dense_mask >> lev) & 1u;
+        const uint32_t R1 = (uint32_t)R + 1u;
+#pragma unroll 4
+        for (int step = 0; step < 8; step++) {
+            const uint32_t q = 4 * step + (lane >> 4);
+            if (q >= queries) continue;
+            const float d = df[q * kDfStride + 2 * lev + f];
+            if (d == 0.0f) continue;
+            // the corner's entry and weight, as level_corners gives them
+            const float sx = pos[3 * q] * R, sy = pos[3 * q + 1] * R, sz = pos[3 * q + 2] * R;
+            const float x0 = fminf(floorf(sx), R - 1.0f), y0 = fminf(floorf(sy), R - 1.0f),
+                        z0 = fminf(floorf(sz), R - 1.0f);
+            const float fx = sx - x0, fy = sy - y0, fz = sz - z0;
+            const uint32_t px = (uint32_t)x0 + cx, py = (uint32_t)y0 + cy, pz = (uint32_t)z0 + cz;
+            const uint32_t h =
+                dense ? px + R1 * (py + R1 * pz) : ((px ^ (py * 2654435761u) ^ (pz * 805459861u)) & (T - 1u));
+            const float w = ((cx ? fx : 1.0f - fx) * (cy ? fy : 1.0f - fy)) * (cz ? fz : 1.0f - fz);
+            atomicAdd(grad + 2 * ((size_t)lev * T + h) + f, w * d);
         }
     }
 }
@@ -290,6 +304,7 @@ __device__ __forceinline__ void dw_step(uint16_t* xs, uint16_t* ds, const u32x4 
 constexpr int kInferQT = kInferQueriesPerWave / 16;
 constexpr int kTrainQT = kTrainQueriesPerWave / 16;
 static_assert(kTrainQT == 2, "the weight-gradient product takes K = 32 queries per chunk");
+static_assert(kStage * sizeof(uint16_t) >= 32 * kDfStride * sizeof(float), "the staging rows hold the feature gradients");
 
 // count = *d_count when d_count is set (device-resident counts), else n.
 __global__ __launch_bounds__(256) void k_nrc_infer(NrcDev P, const float4* __restrict__ q, float4* __restrict__ out,
@@ -427,15 +442,31 @@ __global__ __launch_bounds__(kTrainBlock, 1) void k_nrc_train(NrcDev P, const fl
         f32x4 dx0[2][QT];
         bwd_layer<0, QT>(P.wk, dz, dx0, lane);
 
-        // input-feature gradients -> hash table
+        // input-feature gradients -> hash table, through the staging rows
+        float* df = reinterpret_cast<float*>(xs);
+        float* pos = reinterpret_cast<float*>(ds);
 #pragma unroll
         for (int t = 0; t < QT; t++) {
-            const uint32_t qi = base + 16 * t + r;
-            if (qi >= count) continue;
-            const float df[8] = {dx0[0][t][0], dx0[0][t][1], dx0[0][t][2], dx0[0][t][3],
+            const float d8[8] = {dx0[0][t][0], dx0[0][t][1], dx0[0][t][2], dx0[0][t][3],
                                  dx0[1][t][0], dx0[1][t][1], dx0[1][t][2], dx0[1][t][3]};
-            lane_table_grad(P, q, qi, g, df, grad_table);
+            const int qn = 16 * t + r;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int lev = slot_level(g, j);
+                if (lev < 0) continue;
+                df[qn * kDfStride + 2 * lev] = d8[2 * j];
+                df[qn * kDfStride + 2 * lev + 1] = d8[2 * j + 1];
+            }
+            if (g == 0 && base + qn < count) {
+                const float4 a = q[3 * (size_t)(base + qn)];
+                pos[3 * qn] = clamp01((a.x - P.bmin[0]) * P.binv[0]);
+                pos[3 * qn + 1] = clamp01((a.y - P.bmin[1]) * P.binv[1]);
+                pos[3 * qn + 2] = clamp01((a.z - P.bmin[2]) * P.binv[2]);
+            }
         }
+        wave_sync();
+        wave_table_grad(P, df, pos, min(count - base, (uint32_t)kTrainQueriesPerWave), lane, grad_table);
+        wave_sync();
     }
 
     // loss: one atomic per wave
@@ -446,12 +477,25 @@ __global__ __launch_bounds__(kTrainBlock, 1) void k_nrc_train(NrcDev P, const fl
     for (int j = threadIdx.x; j < kMasterSize; j += kTrainBlock) dst[j] = dW[j];
 }
 
-__global__ void k_mlp_reduce(const float* __restrict__ partial, uint32_t blocks, float* __restrict__ grad_out,
-                             float* __restrict__ master, float* __restrict__ m, float* __restrict__ v, float lr_t) {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= (uint32_t)kMasterSize) return;
-    float s = 0.0f;
-    for (uint32_t b = 0; b < blocks; b++) s += partial[(size_t)b * kMasterSize + j];
+// Sums the blocks' weight gradients, 64 weights per group: wave w of four adds
+// every fourth block's (coalesced, eight loads in flight), then the first
+// adds the four sums.  One thread per weight instead walks all the blocks on
+// a quarter of the chip (256 blocks: 62 us against 9).
+constexpr uint32_t kReduceWeights = 64, kReduceWaves = 4;
+__global__ __launch_bounds__(kReduceWeights * kReduceWaves) void k_mlp_reduce(
+    const float* __restrict__ partial, uint32_t blocks, float* __restrict__ grad_out, float* __restrict__ master,
+    float* __restrict__ m, float* __restrict__ v, float lr_t) {
+    __shared__ float part[kReduceWaves][kReduceWeights];
+    const uint32_t lane = threadIdx.x % kReduceWeights, wave = threadIdx.x / kReduceWeights;
+    const uint32_t j = blockIdx.x * kReduceWeights + lane;
+    static_assert(kMasterSize % kReduceWeights == 0, "every lane has a weight");
+    float t = 0.0f;
+#pragma unroll 8
+    for (uint32_t b = wave; b < blocks; b += kReduceWaves) t += partial[(size_t)b * kMasterSize + j];
+    part[wave][lane] = t;
+    __syncthreads();
+    if (wave != 0) return;
+    const float s = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
     if (m == nullptr) {
         grad_out[j] = s;
         return;
@@ -563,7 +607,8 @@ hipError_t launch_train(const NrcDev& d, const float4* queries, const float4* ta
 
 hipError_t launch_mlp_reduce(const float* partial, uint32_t blocks, float* grad_out, float* master, float* m, float* v,
                              float lr_t, hipStream_t stream) {
-    hipLaunchKernelGGL(k_mlp_reduce, dim3(blocks_for(kMasterSize, 256)), dim3(256), 0, stream, partial, blocks,
+    hipLaunchKernelGGL(k_mlp_reduce, dim3(kMasterSize / kReduceWeights), dim3(kReduceWeights * kReduceWaves), 0, stream,
+                       partial, blocks,
                        grad_out, master, m, v, lr_t);
     return hipGetLastError();
 }
