@@ -75,19 +75,32 @@ __device__ __forceinline__ F3 decode_normal(uint32_t packed) {
 
 struct Pixel {
     float depth;
+    float phi;              // of the depth agreement
     uint32_t material;
+    uint32_t packed_normal;
     F3 normal;
+    float same_normal;      // the normal agreement of an equal normal
 };
 
-// IsHistoryPixelValid: normal agreement ^ 16, same material, depth agreement.
-__device__ __forceinline__ bool history_valid(const TemporalArgs& T, uint32_t idx, const Pixel& c) {
-    const F3 hn = decode_normal(T.hnormal[idx]);
-    const float d = gmax((hn.x * c.normal.x + hn.y * c.normal.y) + hn.z * c.normal.z, 0.0f);
+__device__ __forceinline__ float normal_agreement(F3 hn, F3 n) {
+    const float d = gmax((hn.x * n.x + hn.y * n.y) + hn.z * n.z, 0.0f);
     const float d2 = d * d, d4 = d2 * d2, d8 = d4 * d4;
-    float confidence = d8 * d8;
-    confidence *= uint32_t(T.hmaterial[idx]) != c.material ? 0.0f : 1.0f;
-    const float phi = 16.0f / fabsf(c.depth);
-    confidence *= gmin(1.0f, expf(-fabsf(c.depth - T.hdepth[idx]) * phi));
+    return d8 * d8;
+}
+
+// IsHistoryPixelValid: normal agreement ^ 16, same material, depth agreement.
+// Up to 29 history texels per pixel ask; on a surface that did not move the
+// normals and depths are mostly the pixel's own, which need no square root,
+// divisions and exponential: an equal normal has the agreement computed once
+// per pixel, an equal depth's agreement is 1 (exp(-0), and gmin's 1 where phi
+// is infinite).  Another material's confidence is 0 or NaN, never over 0.1.
+__device__ __forceinline__ bool history_valid(const TemporalArgs& T, uint32_t idx, const Pixel& c) {
+    if (uint32_t(T.hmaterial[idx]) != c.material) return false;
+    const uint32_t packed = T.hnormal[idx];
+    float confidence = c.same_normal;
+    if (packed != c.packed_normal) confidence = normal_agreement(decode_normal(packed), c.normal);
+    const float depth = T.hdepth[idx];
+    if (depth != c.depth) confidence *= gmin(1.0f, expf(-fabsf(c.depth - depth) * c.phi));
     return confidence > 0.1f;
 }
 
@@ -110,14 +123,26 @@ __global__ __launch_bounds__(kTile * kTile) void k_temporal(TemporalArgs T) {
         tile[i] = make_float4(r.x, r.y, r.z, T.depth[idx]);
     }
     __syncthreads();
+    // a tile of one texel value (the sky): every tap has the same colour and
+    // weight, so the sums need neither the taps nor their exponentials
+    const float4 t0 = tile[0];
+    bool same = true;
+    for (int i = int(threadIdx.x); i < kSide * kSide; i += kTile * kTile) {
+        const float4 t = tile[i];
+        same = same && t.x == t0.x && t.y == t0.y && t.z == t0.z && t.w == t0.w;
+    }
+    const bool flat = __syncthreads_and(same) != 0;
     const int lx = int(threadIdx.x) % kTile, ly = int(threadIdx.x) / kTile;
     const int px = int(blockIdx.x) * kTile + lx, py = int(blockIdx.y) * kTile + ly;
     if (px >= int(T.width) || py >= int(T.height)) return;
     const uint32_t idx = uint32_t(py) * T.width + uint32_t(px);
     Pixel c;
     c.depth = T.depth[idx];
+    c.phi = 16.0f / fabsf(c.depth);
     c.material = T.material[idx];
-    c.normal = decode_normal(T.normal[idx]);
+    c.packed_normal = T.normal[idx];
+    c.normal = decode_normal(c.packed_normal);
+    c.same_normal = normal_agreement(c.normal, c.normal);
 
     // ComputeVarianceMinMax: i over x, j over y
     F3 m1 = f3(0.0f, 0.0f, 0.0f), m2 = f3(0.0f, 0.0f, 0.0f);
@@ -126,7 +151,17 @@ __global__ __launch_bounds__(kTile * kTile) void k_temporal(TemporalArgs T) {
     // on the hardware exp2 (GLSL allows 2.5 ulp for a division and
     // 3 + 2 |x| ulp for exp)
     const float inv_phi = 1.0f / gmax(1.0f, fabsf(0.025f * c.depth));
-    for (int i = -kRadius; i <= kRadius; i++)
+    if (flat) {
+        const float w = gmin(1.0f, __expf(-fabsf(c.depth - t0.w) * inv_phi));
+        const F3 a1 = f3(t0.x * w, t0.y * w, t0.z * w);
+        const F3 a2 = f3((t0.x * t0.x) * w, (t0.y * t0.y) * w, (t0.z * t0.z) * w);
+        for (int i = 0; i < (2 * kRadius + 1) * (2 * kRadius + 1); i++) {
+            m1 = f3(m1.x + a1.x, m1.y + a1.y, m1.z + a1.z);
+            m2 = f3(m2.x + a2.x, m2.y + a2.y, m2.z + a2.z);
+            total += w;
+        }
+    }
+    for (int i = -kRadius; i <= kRadius && !flat; i++)
         for (int j = -kRadius; j <= kRadius; j++) {
             const float4 t = tile[(ly + kRadius + j) * kSide + (lx + kRadius + i)];
             const F3 r = f3(t.x, t.y, t.z);
