@@ -306,42 +306,110 @@ constexpr int kTrainQT = kTrainQueriesPerWave / 16;
 static_assert(kTrainQT == 2, "the weight-gradient product takes K = 32 queries per chunk");
 static_assert(kStage * sizeof(uint16_t) >= 32 * kDfStride * sizeof(float), "the staging rows hold the feature gradients");
 
-// count = *d_count when d_count is set (device-resident counts), else n.
-__global__ __launch_bounds__(256) void k_nrc_infer(NrcDev P, const float4* __restrict__ q, float4* __restrict__ out,
-                                                   const uint32_t* __restrict__ d_count, uint32_t n) {
-    constexpr int QT = kInferQT;
-    const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
-    const uint32_t count = d_count ? min(*d_count, n) : n;
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const uint32_t base = wave * (16 * QT);
-    if (base >= count) return;  // wave-uniform
-    u32x4 x0[1][QT];
+// The two features of level `lev` at (x, y, z), as lane_features sums them.
+__device__ __forceinline__ uint32_t level_feature(const NrcDev& P, int lev, float x, float y, float z) {
+    uint32_t idx[8];
+    float w[8];
+    level_corners(P, lev, x, y, z, idx, w);
+    const uint32_t* tab = reinterpret_cast<const uint32_t*>(P.table);
+    uint32_t e[8];
+    if ((P.dense_mask >> lev) & 1u) {  // the two corners along x are neighbours
 #pragma unroll
-    for (int t = 0; t < QT; t++) {
-        const uint32_t qi = base + 16 * t + r;
-        float f[8];
-        lane_features(P, q, qi, qi < count, g, f);
-        x0[0][t] = u32x4{pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3]), pack_bf16(f[4], f[5]), pack_bf16(f[6], f[7])};
+        for (int c = 0; c < 8; c += 2) __builtin_memcpy(&e[c], tab + idx[c], 8);
+    } else {
+#pragma unroll
+        for (int c = 0; c < 8; c++) e[c] = tab[idx[c]];
     }
-    f32x4 z[4][QT];
-    u32x4 h[2][QT];
-    fwd_layer<0, QT>(P.wn, x0, z, lane);
-    relu_pack<QT>(z, h);
-    fwd_layer<1, QT>(P.wn, h, z, lane);
-    relu_pack<QT>(z, h);
-    fwd_layer<2, QT>(P.wn, h, z, lane);
-    relu_pack<QT>(z, h);
-    fwd_layer<3, QT>(P.wn, h, z, lane);
-    relu_pack<QT>(z, h);
-    fwd_layer<4, QT>(P.wn, h, z, lane);
-    relu_pack<QT>(z, h);
-    f32x4 y[1][QT];
-    fwd_layer<5, QT>(P.wn, h, y, lane);
-    if (g == 0) {
+    float f0 = 0.0f, f1 = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        f0 += w[c] * half_to_float(e[c] & 0xffffu);
+        f1 += w[c] * half_to_float(e[c] >> 16);
+    }
+    return pack_bf16(f0, f1);
+}
+
+// Inference, TILES tiles of 64 queries per wave; count = *d_count when
+// d_count is set (device-resident counts), else n.
+//
+// The gathers from the hash table bound it: 12 levels x 8 corners per query,
+// mostly one cache line per two corners.  Taken query by query they spread
+// over the whole table (25 MB at 12 x 2^19 entries), and most of the lines
+// come from outside the XCD's 4 MB L2.  Here a wave takes one level for all
+// of its queries before the next, one query per lane; the waves of the chip
+// start together and move through the levels at about the same pace, so the
+// level in use (2 MB) mostly stays in every L2.  The features wait in LDS as
+// the BF16 pairs that the network's first layer reads.  One wave per block
+// spreads any count evenly over the CUs; two waves per SIMD leave the network
+// its registers, with four (128 registers, spilled) 460,001 queries take
+// 170 us.  460,001 queries: 230 -> 137 us, 100,000: 69 -> 40,
+// 1,000: 26 -> 15.
+template <int TILES>
+__global__ __launch_bounds__(64, 2) void k_nrc_infer(NrcDev P, const float4* __restrict__ q, float4* __restrict__ out,
+                                                      const uint32_t* __restrict__ d_count, uint32_t n) {
+    constexpr int QT = kInferQT;
+    constexpr int kRow = kMaxLevels + 1;  // dwords per query: odd, so that lanes fall on different banks
+    __shared__ uint32_t features[TILES][64 * kRow];
+    const int lane = threadIdx.x, g = lane >> 4, r = lane & 15;
+    const uint32_t count = d_count ? min(*d_count, n) : n;
+    // the tiles that are there, spread over the whole grid
+    if (count == 0) return;
+    const uint32_t per_wave = (count - 1) / (64 * gridDim.x) + 1;  // at most TILES
+    const uint32_t first = blockIdx.x * per_wave * 64;
+    if (first >= count) return;  // wave-uniform
+    float x[TILES], y[TILES], z3[TILES];
+#pragma unroll
+    for (int t = 0; t < TILES; t++) {
+        const uint32_t qi = min(first + 64 * min((uint32_t)t, per_wave - 1) + lane, count - 1);
+        const float4 a = q[3 * (size_t)qi];
+        x[t] = clamp01((a.x - P.bmin[0]) * P.binv[0]);
+        y[t] = clamp01((a.y - P.bmin[1]) * P.binv[1]);
+        z3[t] = clamp01((a.z - P.bmin[2]) * P.binv[2]);
+    }
+#pragma unroll 1
+    for (int lev = 0; lev < kMaxLevels; lev++) {
+#pragma unroll
+        for (int t = 0; t < TILES; t++)
+            if (t == 0 || t < (int)per_wave)  // wave-uniform
+                features[t][lane * kRow + lev] = lev < (int)P.levels ? level_feature(P, lev, x[t], y[t], z3[t]) : 0u;
+    }
+    wave_sync();
+    for (uint32_t tile = 0; tile < per_wave; tile++) {
+        const uint32_t base = first + 64 * tile;
+        if (base >= count) break;  // wave-uniform
+        u32x4 x0[1][QT];
 #pragma unroll
         for (int t = 0; t < QT; t++) {
-            const uint32_t qi = base + 16 * t + r;
-            if (qi < count) out[qi] = make_float4(y[0][t][0], y[0][t][1], y[0][t][2], 0.0f);
+            const uint32_t qi = min(base + 16 * t + r, count - 1);
+            const uint32_t* row = &features[tile][(16 * t + r) * kRow];
+            u32x4 v{row[2 * g], row[2 * g + 1], row[8 + 2 * (g & 1)], row[9 + 2 * (g & 1)]};
+            if (g >= 2) {  // directions, normal, roughness and the constant input
+                const float4 a = q[3 * (size_t)qi], b = q[3 * (size_t)qi + 1], c = q[3 * (size_t)qi + 2];
+                v[2] = g == 2 ? pack_bf16(b.x, b.y) : pack_bf16(c.y, c.z);
+                v[3] = g == 2 ? pack_bf16(b.z, c.x) : pack_bf16(a.w, 1.0f);
+            }
+            x0[0][t] = v;
+        }
+        f32x4 z[4][QT];
+        u32x4 h[2][QT];
+        fwd_layer<0, QT>(P.wn, x0, z, lane);
+        relu_pack<QT>(z, h);
+        fwd_layer<1, QT>(P.wn, h, z, lane);
+        relu_pack<QT>(z, h);
+        fwd_layer<2, QT>(P.wn, h, z, lane);
+        relu_pack<QT>(z, h);
+        fwd_layer<3, QT>(P.wn, h, z, lane);
+        relu_pack<QT>(z, h);
+        fwd_layer<4, QT>(P.wn, h, z, lane);
+        relu_pack<QT>(z, h);
+        f32x4 o[1][QT];
+        fwd_layer<5, QT>(P.wn, h, o, lane);
+        if (g == 0) {
+#pragma unroll
+            for (int t = 0; t < QT; t++) {
+                const uint32_t qi = base + 16 * t + r;
+                if (qi < count) out[qi] = make_float4(o[0][t][0], o[0][t][1], o[0][t][2], 0.0f);
+            }
         }
     }
 }
@@ -583,9 +651,24 @@ static inline uint32_t blocks_for(uint32_t n, uint32_t per) { return (n + per - 
 hipError_t launch_infer(const NrcDev& d, const float4* queries, float4* out, const uint32_t* d_count, uint32_t count,
                         hipStream_t stream) {
     if (count == 0) return hipSuccess;
-    const uint32_t per_block = 256 / 64 * kInferQueriesPerWave;
-    hipLaunchKernelGGL(k_nrc_infer, dim3(blocks_for(count, per_block)), dim3(256), 0, stream, d, queries, out, d_count,
-                       count);
+    // as many tiles per wave as let the whole batch be resident (8 waves per
+    // CU), so that its waves take the levels together: 1 tile per wave at
+    // 460,001 queries takes 221 us, 4 take 137.  A batch of more than that
+    // starts a wave at the first level while others are at the last; six, all
+    // that LDS holds, then gather the most per line: 2,000,000 queries take
+    // 590 us, 675 with four.
+    const uint32_t waves = (uint32_t)device_cu_count() * 8u;
+    const uint32_t tiles = blocks_for(count, 64);
+    const uint32_t per_wave = tiles <= waves ? 1u : (tiles <= 2 * waves ? 2u : (tiles <= 4 * waves ? 4u : 6u));
+    const dim3 grid(blocks_for(tiles, per_wave)), block(64);
+    if (per_wave == 1)
+        hipLaunchKernelGGL((k_nrc_infer<1>), grid, block, 0, stream, d, queries, out, d_count, count);
+    else if (per_wave == 2)
+        hipLaunchKernelGGL((k_nrc_infer<2>), grid, block, 0, stream, d, queries, out, d_count, count);
+    else if (per_wave == 4)
+        hipLaunchKernelGGL((k_nrc_infer<4>), grid, block, 0, stream, d, queries, out, d_count, count);
+    else
+        hipLaunchKernelGGL((k_nrc_infer<6>), grid, block, 0, stream, d, queries, out, d_count, count);
     return hipGetLastError();
 }
 

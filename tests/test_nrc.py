@@ -215,6 +215,26 @@ def test_gpu_nrc_infer_matches_oracle(torch_cuda):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tiles", [1, 2, 4, 6])
+def test_gpu_nrc_infer_is_the_same_at_every_batch_size(torch_cuda, tiles):
+    """A wave takes 1, 2, 4 or 6 tiles of 64 queries by the batch's size; each
+    query's result depends on nothing but the query, so it is the same bit for
+    bit as in a batch of one-tile waves."""
+    print("case nrc infer tiles", tiles, flush=True)
+    torch = torch_cuda
+    g = np.random.default_rng(13)
+    rc = _cache(torch)
+    _set_random(torch, rc, g, _oracle_params())
+    waves = 8 * torch.cuda.get_device_properties(0).multi_processor_count
+    n = {1: 65, 2: 64 * waves + 1, 4: 2 * 64 * waves + 1, 6: 4 * 64 * waves + 1}[tiles]
+    q = torch.from_numpy(rand_queries(g, 4097)).cuda()
+    one = rc.infer(q)
+    q = q.repeat(-(-n // 4097), 1)[:n].contiguous()
+    out = rc.infer(q)
+    assert torch.equal(out, one.repeat(-(-n // 4097), 1)[:n])
+
+
+@pytest.mark.gpu
 def test_gpu_nrc_gradients_match_oracle(torch_cuda):
     print("case nrc gradients", flush=True)
     torch = torch_cuda
