@@ -72,8 +72,8 @@ atlas_rt_status atlas_rt::nrc::train_step(atlas_rt_nrc& N, const float4* queries
     // Adam bias correction folded into the step size
     const double b1t = std::pow(0.9, double(N.step)), b2t = std::pow(0.99, double(N.step));
     const float lr_t = float(double(N.params.learning_rate) * std::sqrt(1.0 - b2t) / (1.0 - b1t));
-    st = hip_check(launch_mlp_reduce(N.partial, blocks, nullptr, N.master, N.m_mlp, N.v_mlp, lr_t, s), "nrc adam");
-    if (st == ATLAS_RT_OK) st = hip_check(launch_pack(N.master, N.wn, N.wk, s), "nrc pack");
+    st = hip_check(launch_mlp_reduce(N.partial, blocks, nullptr, N.master, N.m_mlp, N.v_mlp, N.wn, N.wk, lr_t, s),
+                   "nrc adam");
     if (st == ATLAS_RT_OK)
         st = hip_check(launch_table_adam(N.table32, N.table16, N.m_tab, N.v_tab, N.grad_tab, N.table_params, lr_t, s),
                        "nrc table adam");
@@ -231,7 +231,8 @@ atlas_rt_status atlas_rt_nrc_gradients(atlas_rt_nrc* nrc, const float* d_queries
                                     N.max_blocks, d_grad_table, N.loss, &blocks, s),
                        "nrc train launch");
     if (st == ATLAS_RT_OK)
-        st = hip_check(launch_mlp_reduce(N.partial, blocks, d_grad_mlp, nullptr, nullptr, nullptr, 0.0f, s),
+        st = hip_check(launch_mlp_reduce(N.partial, blocks, d_grad_mlp, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                         0.0f, s),
                        "nrc reduce");
     return st;
 }

@@ -85,9 +85,9 @@ hipError_t launch_train(const NrcDev& d, const float4* queries, const float4* ta
                         uint32_t count, uint32_t slice, uint32_t slices, float* partial, uint32_t max_blocks,
                         float* grad_table, float* loss, uint32_t* blocks, hipStream_t stream);
 // Sum the partials; with m/v set, apply Adam to `master` (lr_t already
-// bias-corrected), else write the sums to grad_out.
+// bias-corrected) and refresh its BF16 copies, else write the sums to grad_out.
 hipError_t launch_mlp_reduce(const float* partial, uint32_t blocks, float* grad_out, float* master, float* m, float* v,
-                             float lr_t, hipStream_t stream);
+                             uint16_t* wn, uint16_t* wk, float lr_t, hipStream_t stream);
 // Adam on the table entries with a non-zero gradient; clears the gradient.
 hipError_t launch_table_adam(float* table32, uint16_t* table16, float* m, float* v, float* grad, uint32_t n,
                              float lr_t, hipStream_t stream);

@@ -45,7 +45,7 @@ __device__ __forceinline__ float half_to_float(uint32_t bits16) {
 __device__ __forceinline__ uint16_t float_to_half(float f) { return __builtin_bit_cast(uint16_t, (_Float16)f); }
 
 __device__ __forceinline__ u32x4 load_frag(const uint16_t* base, int frag, int lane) {
-    return *reinterpret_cast<const u32x4*>(base + ((size_t)frag * 64 + lane) * 8);
+    return *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(base + (size_t)frag * 512) + (uint32_t)lane * 16u);
 }
 
 // ---------------------------------------------------------------------------
@@ -176,6 +176,7 @@ __device__ __forceinline__ void fwd_layer(const uint16_t* __restrict__ wn, const
                                           f32x4 (&z)[kNp[L] / 16][QT], int lane) {
     constexpr int S = kK[L] / 32, T = kNp[L] / 16;
     const uint16_t* w = wn + wn_offset(L);
+    asm volatile("" : "+s"(w));  // a scalar base per layer, not a register pair per fragment kept over the loop
 #pragma unroll
     for (int t = 0; t < T; t++)
 #pragma unroll
@@ -196,6 +197,7 @@ __device__ __forceinline__ void bwd_layer(const uint16_t* __restrict__ wk, const
                                           f32x4 (&dx)[kK[L] / 16][QT], int lane) {
     constexpr int S = nk_cols(L) / 32, T = kK[L] / 16;
     const uint16_t* w = wk + wk_offset(L);
+    asm volatile("" : "+s"(w));  // a scalar base per layer, not a register pair per fragment kept over the loop
 #pragma unroll
     for (int t = 0; t < T; t++)
 #pragma unroll
@@ -263,38 +265,54 @@ __device__ __forceinline__ void stage(uint16_t* st, const u32x4 (&x)[S][QT], int
             }
 }
 
-// dW_L += X_L^T dZ_L over the wave's 32 queries (K of the product), added
-// into the block's LDS gradient.
+// The block's waves share out the 16 x 16 tiles of each layer's weight
+// gradient: each takes kDwTiles neighbours along the outputs.
+constexpr int kTrainWaves = kTrainBlock / 64;
 template <int L>
-__device__ __forceinline__ void dw_layer(const uint16_t* xs, const uint16_t* ds, float* dW, int g, int r) {
-    constexpr int MT = kK[L] / 16, NT = kNp[L] / 16, N = kN[L];
-    float* dst = dW + master_offset(L);
-    u32x4 b[NT];
+constexpr int kDwTiles = (kK[L] / 16) * (kNp[L] / 16) / kTrainWaves;
+template <int L>
+__device__ __forceinline__ int dw_in_tile(int wv) { return wv * kDwTiles<L> / (kNp[L] / 16); }
+template <int L>
+__device__ __forceinline__ int dw_out_tile(int wv) { return wv * kDwTiles<L> % (kNp[L] / 16); }
+
+// acc += the wave's tiles of X_L^T dZ_L over the block's 128 queries: every
+// wave stages its queries' activations and gradients (K of the product), then
+// all of them are read back.  Ends with the staging rows in use.
+template <int L, int S, int QT>
+__device__ __forceinline__ void dw_step(uint16_t (*staging)[2][kStage], const u32x4 (&x)[kK[L] / 32][QT],
+                                        const u32x4 (&dz)[S][QT], f32x4 (&acc)[kDwTiles<L>], int wv, int g, int r) {
+    constexpr int NT = kNp[L] / 16;
+    static_assert(kDwTiles<L> * kTrainWaves == (kK[L] / 16) * NT && (kDwTiles<L> <= NT && NT % kDwTiles<L> == 0),
+                  "whole tiles of one input row per wave");
+    __syncthreads();  // the rows' last readers are done
+    stage<kK[L] / 32, QT>(staging[wv][0], x, g, r);
+    stage<S, QT>(staging[wv][1], dz, g, r);
+    __syncthreads();
+    const int ti = dw_in_tile<L>(wv), to = dw_out_tile<L>(wv);
+#pragma unroll 1  // unrolled, the loads of all steps raise the register count: 331 us, not 327
+    for (int c = 0; c < kTrainWaves; c++) {
+        const u32x4 a = *reinterpret_cast<const u32x4*>(&staging[c][0][(16 * ti + r) * kStride + 8 * g]);
 #pragma unroll
-    for (int to = 0; to < NT; to++) b[to] = *reinterpret_cast<const u32x4*>(ds + (16 * to + r) * kStride + 8 * g);
-#pragma unroll
-    for (int ti = 0; ti < MT; ti++) {
-        const u32x4 a = *reinterpret_cast<const u32x4*>(xs + (16 * ti + r) * kStride + 8 * g);
-#pragma unroll
-        for (int to = 0; to < NT; to++) {
-            const f32x4 d = mfma(a, b[to], f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-            const int out = 16 * to + r;
-            if (out < N) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) atomicAdd(&dst[(16 * ti + 4 * g + i) * N + out], d[i]);
-            }
+        for (int j = 0; j < kDwTiles<L>; j++) {
+            const u32x4 b = *reinterpret_cast<const u32x4*>(&staging[c][1][(16 * (to + j) + r) * kStride + 8 * g]);
+            acc[j] = mfma(a, b, acc[j]);
         }
     }
 }
 
-template <int L, int S, int QT>
-__device__ __forceinline__ void dw_step(uint16_t* xs, uint16_t* ds, const u32x4 (&x)[kK[L] / 32][QT],
-                                        const u32x4 (&dz)[S][QT], float* dW, int g, int r) {
-    stage<kK[L] / 32, QT>(xs, x, g, r);
-    stage<S, QT>(ds, dz, g, r);
-    wave_sync();
-    dw_layer<L>(xs, ds, dW, g, r);
-    wave_sync();
+// Writes the wave's tiles of layer L into the block's weight gradient.
+template <int L>
+__device__ __forceinline__ void dw_store(const f32x4 (&acc)[kDwTiles<L>], float* dst, int wv, int g, int r) {
+    constexpr int N = kN[L];
+#pragma unroll
+    for (int j = 0; j < kDwTiles<L>; j++) {
+        const int out = 16 * (dw_out_tile<L>(wv) + j) + r;
+        if (out < N) {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                dst[master_offset(L) + (16 * dw_in_tile<L>(wv) + 4 * g + i) * N + out] = acc[j][i];
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -415,7 +433,16 @@ __global__ __launch_bounds__(64, 2) void k_nrc_infer(NrcDev P, const float4* __r
 }
 
 // Trains on slice `slice` of `slices` equal slices of the samples; the
-// sample count is *d_count when d_count is set (at most n), else n.
+// sample count is *d_count when d_count is set (at most n), else n.  32
+// queries per wave and step.
+//
+// The activations that the backward pass needs, its accumulators and the
+// wave's tiles of the weight gradient fill the registers of one wave per SIMD
+// (at 256, two waves, they spill: a training step of 65,536 queries takes
+// 344 us and not 327).  The scatter into the table is the largest part, about
+// 200 us.  Adding each step's weight gradient into LDS with atomics took a
+// third of the kernel: the step 486 -> 327 us, 1,024 queries 159 -> 69,
+// 300,000 queries 1,950 -> 1,150.
 __global__ __launch_bounds__(kTrainBlock, 1) void k_nrc_train(NrcDev P, const float4* __restrict__ q,
                                                                const float4* __restrict__ tgt,
                                                                const uint32_t* __restrict__ d_count, uint32_t n,
@@ -423,26 +450,28 @@ __global__ __launch_bounds__(kTrainBlock, 1) void k_nrc_train(NrcDev P, const fl
                                                                float* __restrict__ partial,
                                                                float* __restrict__ grad_table, float* loss) {
     constexpr int QT = kTrainQT;
-    constexpr int kWaves = kTrainBlock / 64;
     const uint32_t total = d_count ? min(*d_count, n) : n;
     const uint32_t first = uint32_t(uint64_t(total) * slice / slices);
     const uint32_t count = uint32_t(uint64_t(total) * (slice + 1) / slices) - first;
     const float inv_norm = count ? 1.0f / (3.0f * float(count)) : 0.0f;
     q += 3 * size_t(first);
     tgt += first;
-    __shared__ float dW[kMasterSize];
-    __shared__ __align__(16) uint16_t staging[kWaves][2][kStage];
-    for (int j = threadIdx.x; j < kMasterSize; j += kTrainBlock) dW[j] = 0.0f;
-    __syncthreads();
+    __shared__ __align__(16) uint16_t staging[kTrainWaves][2][kStage];
 
-    const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15, wv = threadIdx.x >> 6;
-    uint16_t* xs = staging[wv][0];
-    uint16_t* ds = staging[wv][1];
+    const int lane0 = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t chunks = (count + kTrainQueriesPerWave - 1) / kTrainQueriesPerWave;
     float lane_loss = 0.0f;
+    f32x4 w0[kDwTiles<0>]{}, w1[kDwTiles<1>]{}, w2[kDwTiles<2>]{}, w3[kDwTiles<3>]{}, w4[kDwTiles<4>]{},
+        w5[kDwTiles<5>]{};
 
-    for (uint32_t c = blockIdx.x * kWaves + wv; c < chunks; c += gridDim.x * kWaves) {  // wave-uniform
-        const uint32_t base = c * kTrainQueriesPerWave;
+    for (uint32_t c = blockIdx.x * kTrainWaves; c < chunks; c += gridDim.x * kTrainWaves) {  // block-uniform
+        // not loop-invariant to the compiler, which would otherwise keep every
+        // address that follows from the lane in registers, and spill
+        int lane = lane0;
+        asm volatile("" : "+v"(lane));
+        const int g = lane >> 4, r = lane & 15;
+        const uint32_t base = (c + wv) * kTrainQueriesPerWave;  // may lie past the end: no query, no gradient
         // forward, keeping every layer's input as packed bf16
         u32x4 x0[1][QT], h0[2][QT], h1[2][QT], h2[2][QT], h3[2][QT], h4[2][QT];
 #pragma unroll
@@ -491,28 +520,29 @@ __global__ __launch_bounds__(kTrainBlock, 1) void k_nrc_train(NrcDev P, const fl
         // backward
         f32x4 dx[4][QT];
         u32x4 dz[2][QT];
-        dw_step<5, 1, QT>(xs, ds, h4, dz5, dW, g, r);
+        dw_step<5, 1, QT>(staging, h4, dz5, w5, wv, g, r);
         bwd_layer<5, QT>(P.wk, dz5, dx, lane);
         gate_pack<QT>(dx, h4, dz);
-        dw_step<4, 2, QT>(xs, ds, h3, dz, dW, g, r);
+        dw_step<4, 2, QT>(staging, h3, dz, w4, wv, g, r);
         bwd_layer<4, QT>(P.wk, dz, dx, lane);
         gate_pack<QT>(dx, h3, dz);
-        dw_step<3, 2, QT>(xs, ds, h2, dz, dW, g, r);
+        dw_step<3, 2, QT>(staging, h2, dz, w3, wv, g, r);
         bwd_layer<3, QT>(P.wk, dz, dx, lane);
         gate_pack<QT>(dx, h2, dz);
-        dw_step<2, 2, QT>(xs, ds, h1, dz, dW, g, r);
+        dw_step<2, 2, QT>(staging, h1, dz, w2, wv, g, r);
         bwd_layer<2, QT>(P.wk, dz, dx, lane);
         gate_pack<QT>(dx, h1, dz);
-        dw_step<1, 2, QT>(xs, ds, h0, dz, dW, g, r);
+        dw_step<1, 2, QT>(staging, h0, dz, w1, wv, g, r);
         bwd_layer<1, QT>(P.wk, dz, dx, lane);
         gate_pack<QT>(dx, h0, dz);
-        dw_step<0, 2, QT>(xs, ds, x0, dz, dW, g, r);
+        dw_step<0, 2, QT>(staging, x0, dz, w0, wv, g, r);
         f32x4 dx0[2][QT];
         bwd_layer<0, QT>(P.wk, dz, dx0, lane);
 
         // input-feature gradients -> hash table, through the staging rows
-        float* df = reinterpret_cast<float*>(xs);
-        float* pos = reinterpret_cast<float*>(ds);
+        float* df = reinterpret_cast<float*>(staging[wv][0]);
+        float* pos = reinterpret_cast<float*>(staging[wv][1]);
+        __syncthreads();
 #pragma unroll
         for (int t = 0; t < QT; t++) {
             const float d8[8] = {dx0[0][t][0], dx0[0][t][1], dx0[0][t][2], dx0[0][t][3],
@@ -533,16 +563,46 @@ __global__ __launch_bounds__(kTrainBlock, 1) void k_nrc_train(NrcDev P, const fl
             }
         }
         wave_sync();
-        wave_table_grad(P, df, pos, min(count - base, (uint32_t)kTrainQueriesPerWave), lane, grad_table);
+        wave_table_grad(P, df, pos, base < count ? min(count - base, (uint32_t)kTrainQueriesPerWave) : 0u, lane,
+                        grad_table);
         wave_sync();
     }
 
     // loss: one atomic per wave
     for (int m = 32; m >= 1; m >>= 1) lane_loss += __shfl_xor(lane_loss, m, 64);
+    const int lane = lane0, g = lane >> 4, r = lane & 15;
     if (lane == 0 && lane_loss != 0.0f) atomicAdd(loss, lane_loss);
-    __syncthreads();
     float* dst = partial + (size_t)blockIdx.x * kMasterSize;
-    for (int j = threadIdx.x; j < kMasterSize; j += kTrainBlock) dst[j] = dW[j];
+    dw_store<0>(w0, dst, wv, g, r);
+    dw_store<1>(w1, dst, wv, g, r);
+    dw_store<2>(w2, dst, wv, g, r);
+    dw_store<3>(w3, dst, wv, g, r);
+    dw_store<4>(w4, dst, wv, g, r);
+    dw_store<5>(w5, dst, wv, g, r);
+}
+
+// Stores weight j at its places in the forward and the backward fragments
+// (k_pack's inverse; the padding stays as k_pack wrote it).
+__device__ __forceinline__ void put_weight(uint32_t j, uint16_t w, uint16_t* wn, uint16_t* wk) {
+    int L = 0;
+#pragma unroll
+    for (int l = 1; l < kLayers; l++)
+        if (j >= (uint32_t)master_offset(l)) L = l;
+    uint32_t fwd = 0, bwd = 0, local = j;
+#pragma unroll
+    for (int l = 1; l < kLayers; l++)
+        if (L == l) {
+            fwd = wn_offset(l);
+            bwd = wk_offset(l);
+            local = j - master_offset(l);
+        }
+    const uint32_t in = local / kN[L], out = local % kN[L];
+    // value 4 (p / 16) + p % 4 of lane group (p % 16) / 4 is unit p of a K step
+    const auto place = [](uint32_t frag, uint32_t p, uint32_t r) {
+        return (frag * 64 + 16 * ((p & 15) >> 2) + r) * 8 + 4 * (p >> 4) + (p & 3);
+    };
+    wn[fwd + place((out >> 4) * (kK[L] / 32) + (in >> 5), in & 31, out & 15)] = w;
+    wk[bwd + place((in >> 4) * (nk_cols(L) / 32) + (out >> 5), out & 31, in & 15)] = w;
 }
 
 // Sums the blocks' weight gradients, 64 weights per group: wave w of four adds
@@ -552,7 +612,7 @@ __global__ __launch_bounds__(kTrainBlock, 1) void k_nrc_train(NrcDev P, const fl
 constexpr uint32_t kReduceWeights = 64, kReduceWaves = 4;
 __global__ __launch_bounds__(kReduceWeights * kReduceWaves) void k_mlp_reduce(
     const float* __restrict__ partial, uint32_t blocks, float* __restrict__ grad_out, float* __restrict__ master,
-    float* __restrict__ m, float* __restrict__ v, float lr_t) {
+    float* __restrict__ m, float* __restrict__ v, uint16_t* __restrict__ wn, uint16_t* __restrict__ wk, float lr_t) {
     __shared__ float part[kReduceWaves][kReduceWeights];
     const uint32_t lane = threadIdx.x % kReduceWeights, wave = threadIdx.x / kReduceWeights;
     const uint32_t j = blockIdx.x * kReduceWeights + lane;
@@ -572,7 +632,9 @@ __global__ __launch_bounds__(kReduceWeights * kReduceWaves) void k_mlp_reduce(
     const float vj = kBeta2 * v[j] + (1.0f - kBeta2) * s * s;
     m[j] = mj;
     v[j] = vj;
-    master[j] -= lr_t * mj / (sqrtf(vj) + kEps);
+    const float w = master[j] - lr_t * mj / (sqrtf(vj) + kEps);
+    master[j] = w;
+    put_weight(j, (uint16_t)bf16_bits(w), wn, wk);
 }
 
 __global__ void k_table_adam(float* __restrict__ t32, uint16_t* __restrict__ t16, float* __restrict__ m,
@@ -679,7 +741,7 @@ hipError_t launch_train(const NrcDev& d, const float4* queries, const float4* ta
     // with a device-resident count the grid covers the largest slice
     const uint32_t most = d_count ? blocks_for(count, slices) : count;
     const uint32_t chunks = blocks_for(most, kTrainQueriesPerWave);
-    uint32_t nb = blocks_for(chunks, kTrainBlock / 64);
+    uint32_t nb = blocks_for(chunks, kTrainWaves);
     if (nb > max_blocks) nb = max_blocks;
     if (nb == 0) nb = 1;  // an empty slice still writes zero partials
     *blocks = nb;
@@ -689,10 +751,9 @@ hipError_t launch_train(const NrcDev& d, const float4* queries, const float4* ta
 }
 
 hipError_t launch_mlp_reduce(const float* partial, uint32_t blocks, float* grad_out, float* master, float* m, float* v,
-                             float lr_t, hipStream_t stream) {
+                             uint16_t* wn, uint16_t* wk, float lr_t, hipStream_t stream) {
     hipLaunchKernelGGL(k_mlp_reduce, dim3(kMasterSize / kReduceWeights), dim3(kReduceWeights * kReduceWaves), 0, stream,
-                       partial, blocks,
-                       grad_out, master, m, v, lr_t);
+                       partial, blocks, grad_out, master, m, v, wn, wk, lr_t);
     return hipGetLastError();
 }
 

@@ -263,6 +263,48 @@ def test_gpu_nrc_gradients_match_oracle(torch_cuda):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 33, 129])
+def test_gpu_nrc_gradients_of_partial_blocks(torch_cuda, n):
+    """A block's four waves sum the weight gradient of 128 queries together,
+    also where some of them have no query or a part of their 32."""
+    print("case nrc partial blocks", n, flush=True)
+    torch = torch_cuda
+    g = np.random.default_rng(14)
+    P = _oracle_params()
+    rc = _cache(torch)
+    m, tab = _set_random(torch, rc, g, P)
+    q = rand_queries(g, n)
+    t = np.abs(g.normal(size=(n, 4))).astype(np.float32)
+    gm, gt = rc.gradients(torch.from_numpy(q).cuda(), torch.from_numpy(t).cuda())
+    gm, gt = gm.cpu().numpy().astype(np.float64), gt.cpu().numpy().astype(np.float64).reshape(P.levels, P.T, 2)
+    _, gmq, gtq, _ = O.loss_and_grads(P, m, tab, q, t, quantize=True)
+    # a value that lies on a BF16 rounding boundary may round the other way in
+    # the oracle (2^-8 of it), once per layer on its way down six layers
+    assert np.linalg.norm(gm - gmq) < 6 * 2.0**-8 * np.linalg.norm(gmq)
+    assert np.linalg.norm(gt - gtq) < 6 * 2.0**-8 * np.linalg.norm(gtq)
+
+
+@pytest.mark.gpu
+def test_gpu_nrc_gradients_over_several_steps_of_a_block(torch_cuda):
+    """Twice the same samples: every block takes a second step, each sample's
+    gradient is exactly halved, and only the order of the FP32 sums differs."""
+    print("case nrc second step", flush=True)
+    torch = torch_cuda
+    g = np.random.default_rng(15)
+    rc = _cache(torch)
+    _set_random(torch, rc, g, _oracle_params())
+    n = 128 * torch.cuda.get_device_properties(0).multi_processor_count  # one step of the whole grid
+    q = torch.from_numpy(rand_queries(g, n)).cuda()
+    t = torch.from_numpy(np.abs(g.normal(size=(n, 4))).astype(np.float32)).cuda()
+    one = [x.double() for x in rc.gradients(q, t)]
+    two = [x.double() for x in rc.gradients(torch.cat([q, q]), torch.cat([t, t]))]
+    for a, b in zip(one, two):
+        # 1/(3 n) and half of it may round differently: 2^-24 relative, and a
+        # BF16 boundary crossed now and then; the sums differ by their order
+        assert torch.linalg.norm(a - b) < 1e-3 * torch.linalg.norm(a)
+
+
+@pytest.mark.gpu
 def test_gpu_nrc_first_adam_step_closed_form(torch_cuda):
     """From zero moments Adam's first step moves every parameter with a
     non-zero gradient by exactly -lr * sign(g); the loss matches the oracle."""
