@@ -695,7 +695,7 @@ __global__ __launch_bounds__(BLOCK) void k_shadow(WorldDev W, const FrameCtl* __
         vis = L.trans;
     } else {
         do {
-            r = world_step_any<BLOCK, LDS_DEPTH, true>(L, W, ATLAS_RT_MASK_SHADOW, s1.w, S, cap);
+            r = world_step_any<BLOCK, LDS_DEPTH>(L, W, ATLAS_RT_MASK_SHADOW, s1.w, S, cap);
         } while (r == kContinue);
         vis = L.slot >= 0 ? 0.0f : 1.0f;
     }
@@ -735,7 +735,7 @@ __global__ __launch_bounds__(BLOCK) void k_shadow(WorldDev W, const FrameCtl* __
 // launch waits for the slowest path of a bounce before the next bounce
 // starts: the frame's only tail is its slowest whole path.  Lanes that trace
 // closest hits and lanes that trace shadow rays share one step body over
-// opaque worlds (world_step_mixed).  Shading is batched per wave: the wave
+// opaque worlds (world_walk).  Shading is batched per wave: the wave
 // keeps stepping until its busy lanes have all finished a walk (kShadeDiv
 // = 1; 1 / kShadeDiv of them in general), then those lanes shade or add
 // their shadow ray's light together.  Paths refill idle lanes between

@@ -3,7 +3,12 @@
 // Reference: HitClosest / HitAny in BLAS mode (data/shader/raytracer/bvh.hsh:244-267,
 // 411-433), launched one ray per invocation by traceClosest.csh:12-36.
 //
-// Two launch shapes share the per-lane step function of trace_core.h:
+// The engine-exact binary kernels without a register-topped stack (closest and
+// any hit) run on the filtered walk of walk.h, in two launch shapes chosen by
+// launch_walk: one group per batch of rays, or a resident grid that pulls
+// chunks of 64 rays (its rules stand there).  The autotuner's other candidates
+// (register-topped stack, float slab, wide nodes) and the visit counters keep
+// the per-lane step functions of trace_core.h:
 //  * grid: one ray per lane, the whole batch in one grid (the engine's shape);
 //  * persistent: a resident grid of waves pulls rays from a global counter.
 //    Whenever fewer than `refill` lanes of a wave are still traversing, the

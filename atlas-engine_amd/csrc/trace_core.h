@@ -265,51 +265,6 @@ __device__ __forceinline__ int step_closest(const BlasDev& B, LaneState& L, cons
     return kContinue;
 }
 
-// Any-hit step; sets L.slot >= 0 and returns kDone on the first accepted triangle.
-template <int BLOCK, int LDS_DEPTH>
-__device__ __forceinline__ int step_any(const BlasDev& B, LaneState& L, const LaneStack<BLOCK, LDS_DEPTH>& S,
-                                        uint32_t cap, float tmax) {
-    if (L.node >= 0) {
-        const float4* np = B.nodes + 4 * size_t(L.node);
-        const float4 a = ldg4(np), b = ldg4(np + 1), c = ldg4(np + 2), d = ldg4(np + 3);
-        float dl, dr;
-        const bool hl = slab_dist(L.R, a.x, a.y, a.z, a.w, b.x, b.y, tmax, dl);
-        const bool hr = slab_dist(L.R, b.z, b.w, c.x, c.y, c.z, c.w, tmax, dr);
-        const int32_t lp = __float_as_int(d.x), rp = __float_as_int(d.y);
-        if (hl && hr) {
-            if (L.sp >= cap) return kOverflow;
-            S.put(L.sp, rp);
-            L.sp++;
-            L.node = lp;
-        } else if (hl || hr) {
-            L.node = hl ? lp : rp;
-        } else {
-            if (L.sp == 0) return kDone;
-            L.sp--;
-            L.node = S.get(L.sp);
-        }
-        return kContinue;
-    }
-    const int32_t tp = ~L.node;
-    const float4* tr = B.tris + 3 * size_t(tp);
-    const float4 a = ldg4(tr), b = ldg4(tr + 1), c = ldg4(tr + 2);
-    float t, u, v;
-    const bool geo = tri_uvt(L.R, a.x, a.y, a.z, b.x, b.y, b.z, c.x, c.y, c.z, t, u, v);
-    if (geo && t > L.R.tmin && t < tmax) {
-        L.slot = tp;
-        L.hitT = t;
-        return kDone;
-    }
-    if (b.w > 0.0f) {
-        if (L.sp == 0) return kDone;
-        L.sp--;
-        L.node = S.get(L.sp);
-    } else {
-        L.node = ~(tp + 1);
-    }
-    return kContinue;
-}
-
 // ---------------------------------------------------------------------------
 // Generic-stack and wide-node variants (the autotuner's other candidates).
 // Nearest hit distance and the set of reachable triangles are those of the

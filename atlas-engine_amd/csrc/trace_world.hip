@@ -8,8 +8,9 @@
 // as a row vector times mat3x4 (unnormalised direction, so t stays in world
 // units, bvh.hsh:177-180) and selects that instance's BLAS.
 //
-// The BLAS of the current instance is kept in registers; node/triangle steps
-// are the same engine-exact arithmetic as the single-BLAS kernels.
+// Opaque walks run on the filtered two-level walk of world_walk.h, the
+// transparent ones on the step functions of trace_world_core.h; both give the
+// engine's results bit for bit.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
