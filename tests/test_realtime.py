@@ -206,6 +206,39 @@ def test_gpu_realtime_matches_oracle(torch_cuda, spf):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("yaw", [0.0, 35.0, 180.0])
+def test_gpu_resolve_of_flat_tiles(torch_cuda, yaw):
+    """Tiles of one texel value sum it without taps, and unmoved history texels
+    skip the normal and depth agreement: the scene ahead, half of it and only
+    sky, at a ragged size, two frames from one place."""
+    print(f"case resolve flat tiles yaw={yaw}", flush=True)
+    S = _scene()
+    W_, H_ = 83, 61
+    pt = atlas_rt.PathTracer(S["world"], W_, H_, 2, S["mats"], W.sun_light(), env=ENV)
+    pt.set_realtime(samples_per_frame=1)
+    view = atlas_rt.view_matrix((0.0, 15.0, -70.0), yaw, 12.0)
+    vp = atlas_rt.projection_matrix(50.0, W_ / H_) @ view
+    cam = atlas_rt.camera((0.0, 15.0, -70.0), yaw, 12.0, 50.0, W_ / H_)
+    hist = None
+    for f in range(2):
+        pt.render_realtime(cam, atlas_rt.frame_matrices(view, atlas_rt.projection_matrix(50.0, W_ / H_), vp))
+        got = {k: pt.read_realtime(k).cpu().numpy() for k in range(6)}
+        depth, mat = got[_abi.RT_DEPTH], got[_abi.RT_MATERIAL].view(np.uint16)
+        vel, nrm = got[_abi.RT_VELOCITY].view(np.uint32), got[_abi.RT_NORMAL].view(np.uint32)
+        if hist is None:
+            hist = dict(hdepth=np.zeros_like(depth), hnormal=np.zeros_like(nrm), hmaterial=np.zeros_like(mat),
+                        hradiance=np.zeros((H_, W_, 4), np.float32))
+        ref = oracle_rt.temporal(got[_abi.RT_FRAME], depth, vel, nrm, mat, **hist)
+        res = got[_abi.RT_RESOLVED]
+        # the taps' hardware exp2 and division: the bound of the test above
+        assert (np.abs(res - ref) <= 1e-6 + 1e-5 * np.abs(ref)).all(axis=-1).mean() > 0.999
+        hist = dict(hdepth=depth, hnormal=nrm, hmaterial=mat, hradiance=res)
+    if yaw == 180.0:
+        assert len(np.unique(got[_abi.RT_FRAME][..., :3].reshape(-1, 3), axis=0)) == 1
+    pt.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("history", [False, True])
 def test_gpu_realtime_after_world_update(torch_cuda, history):
     """An update between realtime frames re-packs the instances.  Without an
