@@ -1,6 +1,6 @@
 // Radiance-cache kernels for gfx950: fused hash-grid encoding + MLP
 // inference, fused forward/backward training with per-block weight-gradient
-// sums in LDS, and the Adam updates.  Layouts and the lane/unit mapping are
+// sums in registers, and the Adam updates.  Layouts and the lane/unit mapping are
 // described in nrc.h.
 #include <hip/hip_runtime.h>
 

@@ -1,5 +1,6 @@
-// Per-lane BVH2 traversal state machine shared by the BLAS, world and batched
-// kernels.
+// Per-lane BVH2 traversal state machine of the kernels that do not run on the
+// filtered walk (walk.h): visit counters, register-stack, float-slab and
+// wide-node variants, transparency; and the work ranges that all share.
 //
 // Semantics are the engine's HitClosest / HitAny (data/shader/raytracer/bvh.hsh:191-273,
 // 359-441), restated as a step function so that one lane can be refilled with
@@ -11,8 +12,6 @@
 //            at a leaf test its triangles in order, accepting t > tmin and
 //            t < current t (CheckLeafClosest, bvh.hsh:44-72: its extra
 //            t < tmax-at-entry test is implied since t only decreases).
-//   any:     left child first regardless of distance, stop at the first
-//            accepted triangle (CheckLeaf, bvh.hsh:74-104).
 // One step processes one inner node or one triangle.
 #pragma once
 
