@@ -322,15 +322,22 @@ void launch_kernel(atlas_rt_batch_set& s, const BatchLaunch& L, uint32_t grid, u
 // LDS stack rows of the walk: with the staged nodes, 20 waves fit one CU.
 constexpr int kWalkRows = 14;
 
+constexpr uint32_t kWalkLanes = 1280;  // resident, per CU
+
+// Stack rows beyond those in LDS for `lanes` lanes.
+atlas_rt_status walk_spill(atlas_rt_batch_set& s, size_t lanes) {
+    const uint32_t cap = s.max_depth + 1;
+    if (cap < uint32_t(kWalkRows)) return ATLAS_RT_OK;
+    return s.spill.ensure(size_t(cap + 1 - kWalkRows) * lanes * sizeof(int32_t));
+}
+
 template <int BLOCK>
 atlas_rt_status launch_walk(atlas_rt_batch_set& s, const BatchLaunch& L) {
     const uint32_t grid =
-        L.persistent ? uint32_t(device_cu_count()) * (1280u / BLOCK) : (s.total + BLOCK - 1) / BLOCK;
+        L.persistent ? uint32_t(device_cu_count()) * (kWalkLanes / BLOCK) : (s.total + BLOCK - 1) / BLOCK;
     const uint32_t cap = s.max_depth + 1;
-    if (cap >= uint32_t(kWalkRows)) {
-        atlas_rt_status st = s.spill.ensure(size_t(cap + 1 - kWalkRows) * grid * BLOCK * sizeof(int32_t));
-        if (st != ATLAS_RT_OK) return st;
-    }
+    const atlas_rt_status st = walk_spill(s, size_t(grid) * BLOCK);
+    if (st != ATLAS_RT_OK) return st;
     const auto* rays = reinterpret_cast<const float4*>(L.rays);
     auto* hits = reinterpret_cast<float4*>(L.hits);
     int32_t* spill = reinterpret_cast<int32_t*>(s.spill.ptr);
@@ -387,6 +394,10 @@ atlas_rt_status launch_one(atlas_rt_batch_set& s, const BatchLaunch& L) {
 }
 
 }  // namespace
+
+atlas_rt_status reserve_batch(atlas_rt_batch_set& s) {
+    return s.total ? walk_spill(s, size_t(device_cu_count()) * kWalkLanes) : ATLAS_RT_OK;
+}
 
 atlas_rt_status launch_batch(atlas_rt_batch_set& s, const BatchLaunch& L) {
     if (s.total == 0) return ATLAS_RT_OK;
