@@ -35,7 +35,9 @@ BatchLaunch to_launch(const atlas_rt_launch_config& c) {
     L.fslab = (c.kernel & ATLAS_RT_KERNEL_SLAB_FLOAT) != 0;
     L.leaf_batch = (c.kernel & ATLAS_RT_KERNEL_LEAF_BATCH) != 0;
     L.block = c.block ? c.block : 256;
-    L.refill = c.refill ? c.refill : 40;
+    // a wave steps while at least `refill` of its 64 lanes are live: with more
+    // than 64 it would never step
+    L.refill = std::min(c.refill ? c.refill : 40u, 64u);
     return L;
 }
 

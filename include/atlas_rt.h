@@ -388,7 +388,8 @@ typedef struct atlas_rt_batch_set atlas_rt_batch_set;
 typedef struct atlas_rt_launch_config {
     int32_t kernel;       /* ATLAS_RT_KERNEL_*; AUTO = tuned */
     uint32_t block;       /* work-group size: 64, 128 or 256 (0 = default) */
-    uint32_t refill;      /* persistent kernels: refill a wave below this many live lanes (0 = default) */
+    uint32_t refill;      /* persistent kernels: refill a wave below this many live lanes (0 = default, 1 to 64;
+                           * more is taken as 64, the lanes of a wave) */
     uint32_t reserved;
 } atlas_rt_launch_config;
 

@@ -100,3 +100,23 @@ def test_batched_device_count_and_graph_replay(torch_cuda):
         done, untouched = order[:cap], order[cap:]
         assert np.array_equal(rt_cases.hit_bits(got[done]), rt_cases.hit_bits(exp[done])), rep
         assert np.all(got["t"][untouched] == -3.0)
+
+
+@pytest.mark.parametrize("refill", [64, 65, 1 << 20])
+def test_refill_up_to_and_above_the_wave(torch_cuda, refill):
+    """A wave has 64 lanes: a larger threshold is taken as 64.  More rays than
+    the resident lanes, so that every wave is refilled."""
+    print("case batched refill", refill, flush=True)
+    torch = torch_cuda
+    g = W.rng(6, 1)
+    meshes = [W.triangle_soup(n, g) for n in (3000, 200)]
+    counts = [5 * 256 * 256 + 4097, 333]
+    rays = W.random_rays(sum(counts), g)
+    table = [(0, 0, counts[0], 0), (1, counts[0], counts[1], 0)]
+    blases = atlas_rt.build_many(meshes)
+    bs = atlas_rt.BatchSet(blases, table)
+    exp = rt_cases.hit_bits(_expected(meshes, rays, np.array(table)[:, :3], blases))
+    reg = _abi.KERNEL_STACK_REGISTER
+    for kernel in (2, 2 | _abi.KERNEL_LEAF_BATCH, 2 | reg):
+        got = _run(torch, bs, rays, kernel=kernel, block=256, refill=refill)
+        assert np.array_equal(rt_cases.hit_bits(got), exp), kernel
