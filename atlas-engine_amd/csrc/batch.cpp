@@ -212,6 +212,7 @@ atlas_rt_status atlas_rt_batch_destroy(atlas_rt_batch_set* s) {
     for (void* p : {s->d_table, s->d_batches, s->d_prefix})
         if (p) (void)hipFree(p);
     s->spill.release();
+    s->graph_spill.release();
     s->flags.release();
     s->timing.release();
     delete s;
@@ -299,15 +300,19 @@ atlas_rt_status atlas_rt_batch_graph_capture(atlas_rt_batch_set* s, const atlas_
         }
         c = s->best;
     }
-    // Scratch must exist before capture (no allocation inside the graph).
+    // The graph's spill rows must exist before the capture (no allocation
+    // inside it).  An earlier graph keeps its rows until it is destroyed.
+    Scratch rows;
     BatchLaunch L = to_launch(c);
     L.rays = d_rays;
     L.hits = d_hits;
     L.d_count = d_count;
     L.stream = cs;
+    L.spill = &rows;
     atlas_rt_status st = launch_batch(*s, L);
     if (st == ATLAS_RT_OK && hipStreamSynchronize(cs) != hipSuccess) st = fail(ATLAS_RT_E_HIP, "hipStreamSynchronize");
     if (st != ATLAS_RT_OK) {
+        rows.release();
         (void)hipStreamDestroy(cs);
         return st;
     }
@@ -315,8 +320,11 @@ atlas_rt_status atlas_rt_batch_graph_capture(atlas_rt_batch_set* s, const atlas_
     if (s->graph) (void)hipGraphDestroy(s->graph);
     s->graph_exec = nullptr;
     s->graph = nullptr;
+    s->graph_spill.release();
+    s->graph_spill = rows;
     hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) {
+        L.spill = &s->graph_spill;
         st = launch_batch(*s, L);
         hipError_t e2 = hipStreamEndCapture(cs, &s->graph);
         if (st == ATLAS_RT_OK && e2 != hipSuccess) st = hip_fail(e2, "hipStreamEndCapture");

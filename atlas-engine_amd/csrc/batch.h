@@ -30,6 +30,7 @@ struct BatchLaunch {
     uint32_t block = 256;
     uint32_t refill = 40;
     hipStream_t stream = nullptr;
+    Scratch* spill = nullptr;  // stack spill rows other than the set's own
 };
 
 }  // namespace atlas_rt
@@ -55,6 +56,9 @@ struct atlas_rt_batch_set {
     // Captured graph.
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
+    // Its stack spill rows: the set's own are replaced when a later launch
+    // needs more, and the graph keeps their address.
+    atlas_rt::Scratch graph_spill;
 
     atlas_rt::BatchDev dev() const {
         atlas_rt::BatchDev d;

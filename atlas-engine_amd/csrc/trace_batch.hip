@@ -303,6 +303,9 @@ struct Rows {
     static constexpr int value = BLOCK >= 256 ? 24 : 32;
 };
 
+// The stack spill rows of a launch: the set's, or a captured graph's own.
+Scratch& spill_of(atlas_rt_batch_set& s, const BatchLaunch& L) { return L.spill ? *L.spill : s.spill; }
+
 template <int BLOCK, int NODE_W, bool REG, bool FLOAT_SLAB = false, int LEAF_DIV = 0>
 void launch_kernel(atlas_rt_batch_set& s, const BatchLaunch& L, uint32_t grid, uint32_t cap) {
     constexpr int D = Rows<BLOCK>::value;
@@ -311,12 +314,12 @@ void launch_kernel(atlas_rt_batch_set& s, const BatchLaunch& L, uint32_t grid, u
         hipLaunchKernelGGL((k_batch_persistent<BLOCK, D, NODE_W, REG, FLOAT_SLAB, LEAF_DIV>), dim3(grid), dim3(BLOCK), 0,
                            L.stream, s.dev(),
                            L.d_count, reinterpret_cast<const float4*>(L.rays), reinterpret_cast<float4*>(L.hits),
-                           reinterpret_cast<int32_t*>(s.spill.ptr), cap, ctl, L.refill);
+                           reinterpret_cast<int32_t*>(spill_of(s, L).ptr), cap, ctl, L.refill);
     else
         hipLaunchKernelGGL((k_batch_grid<BLOCK, D, NODE_W, REG, FLOAT_SLAB>), dim3(grid), dim3(BLOCK), 0, L.stream,
                            s.dev(),
                            L.d_count, reinterpret_cast<const float4*>(L.rays), reinterpret_cast<float4*>(L.hits),
-                           reinterpret_cast<int32_t*>(s.spill.ptr), cap, ctl);
+                           reinterpret_cast<int32_t*>(spill_of(s, L).ptr), cap, ctl);
 }
 
 // LDS stack rows of the walk: with the staged nodes, 20 waves fit one CU.
@@ -325,10 +328,10 @@ constexpr int kWalkRows = 14;
 constexpr uint32_t kWalkLanes = 1280;  // resident, per CU
 
 // Stack rows beyond those in LDS for `lanes` lanes.
-atlas_rt_status walk_spill(atlas_rt_batch_set& s, size_t lanes) {
+atlas_rt_status walk_spill(const atlas_rt_batch_set& s, Scratch& spill, size_t lanes) {
     const uint32_t cap = s.max_depth + 1;
     if (cap < uint32_t(kWalkRows)) return ATLAS_RT_OK;
-    return s.spill.ensure(size_t(cap + 1 - kWalkRows) * lanes * sizeof(int32_t));
+    return spill.ensure(size_t(cap + 1 - kWalkRows) * lanes * sizeof(int32_t));
 }
 
 template <int BLOCK>
@@ -336,11 +339,11 @@ atlas_rt_status launch_walk(atlas_rt_batch_set& s, const BatchLaunch& L) {
     const uint32_t grid =
         L.persistent ? uint32_t(device_cu_count()) * (kWalkLanes / BLOCK) : (s.total + BLOCK - 1) / BLOCK;
     const uint32_t cap = s.max_depth + 1;
-    const atlas_rt_status st = walk_spill(s, size_t(grid) * BLOCK);
+    const atlas_rt_status st = walk_spill(s, spill_of(s, L), size_t(grid) * BLOCK);
     if (st != ATLAS_RT_OK) return st;
     const auto* rays = reinterpret_cast<const float4*>(L.rays);
     auto* hits = reinterpret_cast<float4*>(L.hits);
-    int32_t* spill = reinterpret_cast<int32_t*>(s.spill.ptr);
+    int32_t* spill = reinterpret_cast<int32_t*>(spill_of(s, L).ptr);
     uint32_t* ctl = reinterpret_cast<uint32_t*>(s.flags.ptr);
     if (!L.persistent)
         hipLaunchKernelGGL((k_batch_walk<BLOCK, kWalkRows, false, 0>), dim3(grid), dim3(BLOCK), 0, L.stream, s.dev(),
@@ -369,7 +372,7 @@ atlas_rt_status launch_one(atlas_rt_batch_set& s, const BatchLaunch& L) {
     }
     const uint32_t cap = variant_cap(L.node_w, s.max_depth + 1, s.max_cap4, s.max_cap8);
     if (cap > uint32_t(D)) {
-        atlas_rt_status st = s.spill.ensure(size_t(cap - D) * threads * sizeof(int32_t));
+        atlas_rt_status st = spill_of(s, L).ensure(size_t(cap - D) * threads * sizeof(int32_t));
         if (st != ATLAS_RT_OK) return st;
     }
     if (!L.persistent && L.node_w != 2)
@@ -396,7 +399,7 @@ atlas_rt_status launch_one(atlas_rt_batch_set& s, const BatchLaunch& L) {
 }  // namespace
 
 atlas_rt_status reserve_batch(atlas_rt_batch_set& s) {
-    return s.total ? walk_spill(s, size_t(device_cu_count()) * kWalkLanes) : ATLAS_RT_OK;
+    return s.total ? walk_spill(s, s.spill, size_t(device_cu_count()) * kWalkLanes) : ATLAS_RT_OK;
 }
 
 atlas_rt_status launch_batch(atlas_rt_batch_set& s, const BatchLaunch& L) {

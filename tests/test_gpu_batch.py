@@ -120,3 +120,37 @@ def test_refill_up_to_and_above_the_wave(torch_cuda, refill):
     for kernel in (2, 2 | _abi.KERNEL_LEAF_BATCH, 2 | reg):
         got = _run(torch, bs, rays, kernel=kernel, block=256, refill=refill)
         assert np.array_equal(rt_cases.hit_bits(got), exp), kernel
+
+
+def test_graph_replays_after_larger_launches_of_its_set(torch_cuda):
+    """A captured graph keeps its own stack spill rows: a later launch of the
+    set that needs more rows than the resident lanes (one ray per lane, more
+    rays than lanes) replaces the set's, and the replays stay right.  The trees
+    are 14 and more levels deep, and 80."""
+    print("case batched graph after a larger launch", flush=True)
+    torch = torch_cuda
+    g = W.rng(6, 2)
+    verts = W.triangle_soup(5000, g)
+    chain_nodes, chain_tris, chain_rays = rt_cases.chain_tree(80)
+    blases = [atlas_rt.Blas.build(verts), atlas_rt.Blas.create(chain_nodes, chain_tris)]
+    assert blases[0].info()[2] >= 14
+    n = 5 * 256 * 256 + 4097
+    rays = np.concatenate([W.random_rays(n, g), chain_rays])
+    table = [(0, 0, n, 0), (1, n, len(chain_rays), 0)]
+    exp = rt_cases.hit_bits(_expected([], rays, np.array(table)[:, :3], blases))
+    d_rays = torch.from_numpy(rays.view(np.float32).reshape(-1, 8).copy()).cuda()
+    for kernel in (2 | _abi.KERNEL_LEAF_BATCH, 2 | _abi.KERNEL_STACK_REGISTER):
+        bs = atlas_rt.BatchSet(blases, table)
+        d_hits = torch.zeros((len(rays), 4), dtype=torch.float32, device="cuda")
+        bs.graph_capture(d_rays, d_hits, None, kernel=kernel, block=256, refill=32)
+        other = _run(torch, bs, rays, kernel=_abi.KERNEL_BVH2_EXACT, block=64)
+        assert np.array_equal(rt_cases.hit_bits(other), exp), kernel
+        for rep in range(3):
+            d_hits.fill_(-3.0)
+            torch.cuda.synchronize()
+            bs.graph_launch()
+            torch.cuda.synchronize()
+            got = d_hits.cpu().numpy().view(atlas_rt.HIT_DTYPE).reshape(-1)
+            assert np.array_equal(rt_cases.hit_bits(got), exp), (kernel, rep)
+            if rep == 1:  # a second capture takes the first one's place
+                bs.graph_capture(d_rays, d_hits, None, kernel=kernel, block=64, refill=32)
