@@ -72,8 +72,5 @@ struct atlas_rt_batch_set {
 };
 
 namespace atlas_rt {
-// Stack spill rows of the resident walk, laid out with the set: allocated by
-// the first trace they made a new set's first 250,000 rays take 790 us, not 460.
-atlas_rt_status reserve_batch(atlas_rt_batch_set& s);
 atlas_rt_status launch_batch(atlas_rt_batch_set& s, const BatchLaunch& L);
 }

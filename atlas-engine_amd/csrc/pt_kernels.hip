@@ -922,8 +922,8 @@ __global__ __launch_bounds__(kFrameBlock, OCC) void k_frame_persistent(ShadeArgs
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const LaneStack<kFrameBlock, kFrameLds> S{lds, spill, tid, blockIdx.x * kFrameBlock + tid,
                                               gridDim.x * kFrameBlock};
-    using Stack = WalkStack<kFrameBlock, kFrameLds>;
-    const Stack SW(lds, spill, blockIdx.x * kFrameBlock + tid, gridDim.x * kFrameBlock, cap);
+    using Stack = WalkStack<kFrameBlock, kFrameLds, 0>;
+    const Stack SW(lds, nullptr, spill, blockIdx.x * kFrameBlock + tid, gridDim.x * kFrameBlock, cap);
     FrameCtl* const ctl0 = A.ctl;  // frame f's seeds and counts in ctl0[f]; ctl0[0].pull counts paths
     const WorldDev W = A.world;
     const AlphaArgs& AA = A.alpha;

@@ -176,7 +176,7 @@ __global__ __launch_bounds__(BLOCK) void k_batch_grid(BatchDev D, const uint32_t
 // that refill below `refill` live lanes from the per-XCD ranges, their node
 // records staged through LDS while work is left, or one work item per lane.
 // LEAF_DIV: triangle steps once 1 / LEAF_DIV of the live lanes wait at a leaf.
-template <int BLOCK, int ROWS, bool PULL, int LEAF_DIV>
+template <int BLOCK, int ROWS, int OWN, bool PULL, int LEAF_DIV>
 __global__ __launch_bounds__(BLOCK, 5) void k_batch_walk(BatchDev D, const uint32_t* __restrict__ d_count,
                                                          const float4* __restrict__ rays, float4* __restrict__ hits,
                                                          int32_t* __restrict__ spill, uint32_t cap,
@@ -184,10 +184,11 @@ __global__ __launch_bounds__(BLOCK, 5) void k_batch_walk(BatchDev D, const uint3
     __shared__ int32_t lds[ROWS * BLOCK];
     __shared__ __align__(16) char staged[PULL ? (BLOCK / kWave) * NodeStage::kBytes : 16];
     const NodeStage stage(staged);
-    using Stack = WalkStack<BLOCK, ROWS>;
+    using Stack = WalkStack<BLOCK, ROWS, OWN>;
     const uint32_t count = d_count ? min(*d_count, D.total) : D.total;
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const Stack S(lds, spill, blockIdx.x * BLOCK + threadIdx.x, gridDim.x * BLOCK, cap);
+    int32_t own[OWN];
+    const Stack S(lds, own, spill, blockIdx.x * BLOCK + threadIdx.x, gridDim.x * BLOCK, cap);
     constexpr uint32_t kNone = 0xFFFFFFFFu;
     Walk w;
     w.node = kEnd;
@@ -327,32 +328,27 @@ constexpr int kWalkRows = 14;
 
 constexpr uint32_t kWalkLanes = 1280;  // resident, per CU
 
-// Stack rows beyond those in LDS for `lanes` lanes.
-atlas_rt_status walk_spill(const atlas_rt_batch_set& s, Scratch& spill, size_t lanes) {
-    const uint32_t cap = s.max_depth + 1;
-    if (cap < uint32_t(kWalkRows)) return ATLAS_RT_OK;
-    return spill.ensure(size_t(cap + 1 - kWalkRows) * lanes * sizeof(int32_t));
-}
-
 template <int BLOCK>
 atlas_rt_status launch_walk(atlas_rt_batch_set& s, const BatchLaunch& L) {
     const uint32_t grid =
         L.persistent ? uint32_t(device_cu_count()) * (kWalkLanes / BLOCK) : (s.total + BLOCK - 1) / BLOCK;
     const uint32_t cap = s.max_depth + 1;
-    const atlas_rt_status st = walk_spill(s, spill_of(s, L), size_t(grid) * BLOCK);
-    if (st != ATLAS_RT_OK) return st;
+    if (const size_t bytes = walk_spill_bytes(cap, kWalkRows + kOwnRows, size_t(grid) * BLOCK)) {
+        const atlas_rt_status st = spill_of(s, L).ensure(bytes);
+        if (st != ATLAS_RT_OK) return st;
+    }
     const auto* rays = reinterpret_cast<const float4*>(L.rays);
     auto* hits = reinterpret_cast<float4*>(L.hits);
     int32_t* spill = reinterpret_cast<int32_t*>(spill_of(s, L).ptr);
     uint32_t* ctl = reinterpret_cast<uint32_t*>(s.flags.ptr);
     if (!L.persistent)
-        hipLaunchKernelGGL((k_batch_walk<BLOCK, kWalkRows, false, 0>), dim3(grid), dim3(BLOCK), 0, L.stream, s.dev(),
+        hipLaunchKernelGGL((k_batch_walk<BLOCK, kWalkRows, kOwnRows, false, 0>), dim3(grid), dim3(BLOCK), 0, L.stream, s.dev(),
                            L.d_count, rays, hits, spill, cap, ctl, L.refill);
     else if (L.leaf_batch)
-        hipLaunchKernelGGL((k_batch_walk<BLOCK, kWalkRows, true, kLeafDiv>), dim3(grid), dim3(BLOCK), 0, L.stream,
+        hipLaunchKernelGGL((k_batch_walk<BLOCK, kWalkRows, kOwnRows, true, kLeafDiv>), dim3(grid), dim3(BLOCK), 0, L.stream,
                            s.dev(), L.d_count, rays, hits, spill, cap, ctl, L.refill);
     else
-        hipLaunchKernelGGL((k_batch_walk<BLOCK, kWalkRows, true, 0>), dim3(grid), dim3(BLOCK), 0, L.stream, s.dev(),
+        hipLaunchKernelGGL((k_batch_walk<BLOCK, kWalkRows, kOwnRows, true, 0>), dim3(grid), dim3(BLOCK), 0, L.stream, s.dev(),
                            L.d_count, rays, hits, spill, cap, ctl, L.refill);
     ATLAS_HIP_TRY(hipGetLastError());
     return ATLAS_RT_OK;
@@ -397,10 +393,6 @@ atlas_rt_status launch_one(atlas_rt_batch_set& s, const BatchLaunch& L) {
 }
 
 }  // namespace
-
-atlas_rt_status reserve_batch(atlas_rt_batch_set& s) {
-    return s.total ? walk_spill(s, s.spill, size_t(device_cu_count()) * kWalkLanes) : ATLAS_RT_OK;
-}
 
 atlas_rt_status launch_batch(atlas_rt_batch_set& s, const BatchLaunch& L) {
     if (s.total == 0) return ATLAS_RT_OK;

@@ -230,8 +230,8 @@ __global__ __launch_bounds__(kBeginBlock) void k_walk_begin(BlasDev B, const flo
 // refill load beside the hit records of the rays they replace.
 enum class Shape { kOnce, kPull };
 
-template <int BLOCK, int ROWS, bool ANY, Shape SHAPE, int LEAF_DIV>
-__global__ __launch_bounds__(BLOCK, ROWS > 14 ? 3 : 5) void k_blas_walk(BlasDev B, const float4* __restrict__ rays,
+template <int BLOCK, int ROWS, int OWN, bool ANY, Shape SHAPE, int LEAF_DIV>
+__global__ __launch_bounds__(BLOCK, SHAPE == Shape::kPull && ROWS > 14 ? 3 : 5) void k_blas_walk(BlasDev B, const float4* __restrict__ rays,
                                                         void* __restrict__ out, int32_t* __restrict__ slots,
                                                         uint32_t count, int32_t* __restrict__ spill, uint32_t cap,
                                                         uint32_t* __restrict__ ctl, uint32_t per_wave, bool chosen) {
@@ -240,9 +240,10 @@ __global__ __launch_bounds__(BLOCK, ROWS > 14 ? 3 : 5) void k_blas_walk(BlasDev 
     __shared__ int32_t lds[ROWS * BLOCK];
     __shared__ __align__(16) char staged[kPulls ? (BLOCK / kWave) * NodeStage::kBytes : 16];
     const NodeStage stage(staged);
-    using Stack = WalkStack<BLOCK, ROWS>;
+    using Stack = WalkStack<BLOCK, ROWS, OWN>;
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const Stack S(lds, spill, blockIdx.x * BLOCK + threadIdx.x, gridDim.x * BLOCK, cap);
+    int32_t own[OWN ? OWN : 1];
+    const Stack S(lds, own, spill, blockIdx.x * BLOCK + threadIdx.x, gridDim.x * BLOCK, cap);
     constexpr uint32_t kNone = 0xFFFFFFFFu;
     Walk w;
     w.node = kEnd;
@@ -381,21 +382,19 @@ static atlas_rt_status ensure_flags(atlas_rt_blas& blas) {
 
 constexpr int kWalkBlock = 256;
 // LDS stack rows: with the staged nodes, five groups of resident waves fit
-// one CU (14 KB + 16.3 KB each).
+// one CU (14 KB + 16.3 KB each); of the waves that run once, as many as the
+// registers allow (20 of 7.7 KB each, for any hit 28 of 5.6 KB).
 constexpr int kWalkRows = 14;
+template <bool ANY>
+constexpr int kOnceRows = ANY ? 22 : 30;
 constexpr uint32_t kWalkGroups = 5;
 
 // Launches below this many rays run once, with as many rays per wave as give
 // every CU eight waves: a wave's step takes as long as its slowest lane's
 // memory access, and all of its lanes' accesses after one another (5,003 rays
 // 0.111 -> 0.093 ms, 16,384 rays 0.194 -> 0.166 ms against 64 per wave).
-constexpr uint32_t kOnceRays = 65536;
+constexpr uint32_t kChooseRays = 65536;
 inline uint32_t rays_per_wave(uint32_t count) { return std::min(64u, (count + 2047u) / 2048u); }
-
-// Spill rows of a walk kernel: entries 1 .. cap, of which ROWS - 1 in LDS.
-inline size_t walk_spill_bytes(uint32_t cap, uint32_t rows, size_t threads) {
-    return cap >= rows ? size_t(cap + 1 - rows) * threads * sizeof(int32_t) : 0;
-}
 
 struct WalkArgs {
     BlasDev B;
@@ -409,19 +408,29 @@ struct WalkArgs {
     hipStream_t stream;
 };
 
+// Without own stack rows where the tree is shallow enough: a kernel that has
+// scratch memory takes 0.2 to 0.4 us longer to launch (37 rays on 1,024
+// triangles: 24.1 us, not 23.9; launches of 36.8 us: 37.3).
 template <bool ANY>
 static void walk_once(const WalkArgs& a, uint32_t groups, uint32_t per_wave, bool chosen) {
-    hipLaunchKernelGGL((k_blas_walk<64, kWalkRows, ANY, Shape::kOnce, 0>), dim3(groups), dim3(64), 0, a.stream, a.B,
-                       a.rays, a.out, a.slots, a.count, a.spill, a.cap, a.ctl, per_wave, chosen);
+    const auto launch = [&](auto own) {
+        hipLaunchKernelGGL((k_blas_walk<64, kOnceRows<ANY>, decltype(own)::value, ANY, Shape::kOnce, 0>), dim3(groups),
+                           dim3(64), 0, a.stream, a.B, a.rays, a.out, a.slots, a.count, a.spill, a.cap, a.ctl, per_wave,
+                           chosen);
+    };
+    if (a.cap < uint32_t(kOnceRows<ANY>))
+        launch(std::integral_constant<int, 0>{});
+    else
+        launch(std::integral_constant<int, kOwnRows>{});
 }
 
-template <bool ANY, int ROWS = kWalkRows>
+template <bool ANY, int ROWS = kWalkRows, int OWN = kOwnRows>
 static void walk_pull(const WalkArgs& a, bool leaf_batch, uint32_t groups, bool chosen) {
     if (leaf_batch)
-        hipLaunchKernelGGL((k_blas_walk<kWalkBlock, ROWS, ANY, Shape::kPull, kLeafDiv>), dim3(groups), dim3(kWalkBlock),
+        hipLaunchKernelGGL((k_blas_walk<kWalkBlock, ROWS, OWN, ANY, Shape::kPull, kLeafDiv>), dim3(groups), dim3(kWalkBlock),
                            0, a.stream, a.B, a.rays, a.out, a.slots, a.count, a.spill, a.cap, a.ctl, 64u, chosen);
     else
-        hipLaunchKernelGGL((k_blas_walk<kWalkBlock, ROWS, ANY, Shape::kPull, 0>), dim3(groups), dim3(kWalkBlock), 0,
+        hipLaunchKernelGGL((k_blas_walk<kWalkBlock, ROWS, OWN, ANY, Shape::kPull, 0>), dim3(groups), dim3(kWalkBlock), 0,
                            a.stream, a.B, a.rays, a.out, a.slots, a.count, a.spill, a.cap, a.ctl, 64u, chosen);
 }
 
@@ -433,15 +442,19 @@ enum class WalkPlan { kAuto, kOnce, kPull, kPullLeafBatch };
 
 template <bool ANY>
 static atlas_rt_status launch_walk(atlas_rt_blas& blas, const TraceLaunch& L, WalkPlan plan) {
-    const bool choose = plan == WalkPlan::kAuto && L.count >= kOnceRays;
-    const bool pull = choose || plan == WalkPlan::kPull || plan == WalkPlan::kPullLeafBatch;
+    const uint32_t cap = limit_cap(blas.max_depth + 1, blas.stack_limit);
+    // a tree so deep that a wave per 64 rays would need spill rows keeps to the
+    // resident shape, whose lanes are fewer than a large batch's rays
+    const bool large = plan == WalkPlan::kAuto && L.count >= kChooseRays;
+    const bool choose = large && walk_spill_bytes(cap, kOnceRows<ANY> + kOwnRows, 1) == 0;
+    const bool pull = large || plan == WalkPlan::kPull || plan == WalkPlan::kPullLeafBatch;
     const bool once = choose || !pull;
     const uint32_t per_wave = once && !choose && plan == WalkPlan::kAuto ? rays_per_wave(L.count) : 64u;
     const uint32_t once_groups = (L.count - 1) / per_wave + 1;
     const uint32_t pull_groups = uint32_t(device_cu_count()) * kWalkGroups;
-    const uint32_t cap = limit_cap(blas.max_depth + 1, blas.stack_limit);
-    const size_t threads = std::max(once ? size_t(once_groups) * 64 : 0, pull ? size_t(pull_groups) * kWalkBlock : 0);
-    const size_t spill_bytes = walk_spill_bytes(cap, kWalkRows, threads);
+    const size_t spill_bytes =
+        std::max(once ? walk_spill_bytes(cap, kOnceRows<ANY> + kOwnRows, size_t(once_groups) * 64) : 0,
+                 pull ? walk_spill_bytes(cap, kWalkRows + kOwnRows, size_t(pull_groups) * kWalkBlock) : 0);
     atlas_rt_status st = ATLAS_RT_OK;
     if (spill_bytes) st = blas.spill.ensure(spill_bytes);
     if (st == ATLAS_RT_OK) st = ensure_flags(blas);
@@ -652,7 +665,7 @@ atlas_rt_status launch_blas_closest_noalloc(const atlas_rt_blas& blas, const Tra
                          spill,  cap,                                    ctl,    L.stream};
         static_assert(kPLdsDepth == 24, "the refusal above is the spill bound");
         const uint32_t walk_groups = uint32_t(device_cu_count()) * 3;
-        walk_pull<false, kPLdsDepth>(a, leaf_batch, walk_groups, false);
+        walk_pull<false, kPLdsDepth, 0>(a, leaf_batch, walk_groups, false);
     } else if (leaf_batch) {
         if (fslab)
             reg ? launch_persistent<2, true, true, kLeafDiv>(B, L, groups, spill, cap, ctl)

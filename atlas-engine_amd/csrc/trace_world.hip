@@ -25,10 +25,9 @@ namespace atlas_rt {
 namespace {
 
 // Stack rows in LDS of the walk kernels, one wave of 64 per group: as many as
-// 20 groups per CU, all that the registers allow, leave room for.  20 rows
-// time the same, but the first trace of more worlds has to allocate spill rows
-// for every lane of the grid (first pass of 256 instances, 1280x720: 229 us
-// against 300 to 800).
+// 20 groups per CU, all that the registers allow, leave room for.  Worlds that
+// need no more run without own rows: a kernel that has scratch memory takes
+// 0.2 to 0.4 us longer to launch.
 constexpr int kWalkRows = 30;
 
 // The lane's ray of a group that takes `per_wave` rays, or ~0.
@@ -38,15 +37,16 @@ __device__ __forceinline__ uint32_t lane_ray(uint32_t per_wave, uint32_t count) 
 }
 
 // Compact ray in (32 B) -> refined hit (16 B) + caller instance index.
-template <int ROWS>
+template <int ROWS, int OWN>
 __global__ __launch_bounds__(64, 5) void k_world_closest_rays(WorldDev W, const float4* __restrict__ rays,
                                                               float4* __restrict__ hits, int32_t* __restrict__ inst_out,
                                                               uint32_t count, uint32_t mask,
                                                               int32_t* __restrict__ spill, uint32_t cap,
                                                               uint32_t* __restrict__ ctl, uint32_t per_wave) {
     __shared__ int32_t lds[ROWS * 64];
-    using Stack = WalkStack<64, ROWS>;
-    const Stack S(lds, spill, blockIdx.x * 64 + threadIdx.x, gridDim.x * 64, cap);
+    using Stack = WalkStack<64, ROWS, OWN>;
+    int32_t own[OWN ? OWN : 1];
+    const Stack S(lds, own, spill, blockIdx.x * 64 + threadIdx.x, gridDim.x * 64, cap);
     const uint32_t ray = lane_ray(per_wave, count);
     float4 r0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), r1 = r0;
     if (ray != ~0u) {
@@ -75,14 +75,15 @@ __global__ __launch_bounds__(64, 5) void k_world_closest_rays(WorldDev W, const 
     if (inst_out) inst_out[ray] = caller_inst;
 }
 
-template <int ROWS, bool RESTORE_ALWAYS>
+template <int ROWS, int OWN, bool RESTORE_ALWAYS>
 __global__ __launch_bounds__(64, 5) void k_world_any_rays(WorldDev W, const float4* __restrict__ rays,
                                                           uint32_t* __restrict__ out, uint32_t count, uint32_t mask,
                                                           int32_t* __restrict__ spill, uint32_t cap,
                                                           uint32_t* __restrict__ ctl, uint32_t per_wave) {
     __shared__ int32_t lds[ROWS * 64];
-    using Stack = WalkStack<64, ROWS>;
-    const Stack S(lds, spill, blockIdx.x * 64 + threadIdx.x, gridDim.x * 64, cap);
+    using Stack = WalkStack<64, ROWS, OWN>;
+    int32_t own[OWN ? OWN : 1];
+    const Stack S(lds, own, spill, blockIdx.x * 64 + threadIdx.x, gridDim.x * 64, cap);
     const uint32_t ray = lane_ray(per_wave, count);
     float4 r0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), r1 = r0;
     if (ray != ~0u) {
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(64, 5) void k_world_any_rays(WorldDev W, const floa
 
 // Engine-shaped PackedRay kernels (traceClosest.csh:12-36).  The live ray
 // count is read on the device.
-template <int ROWS>
+template <int ROWS, int OWN>
 __global__ __launch_bounds__(64, 5) void k_world_closest_packed(WorldDev W, const float4* __restrict__ in,
                                                                 float4* __restrict__ out,
                                                                 const uint32_t* __restrict__ d_count,
@@ -108,8 +109,9 @@ __global__ __launch_bounds__(64, 5) void k_world_closest_packed(WorldDev W, cons
                                                                 uint32_t cap, uint32_t* __restrict__ ctl,
                                                                 uint32_t per_wave) {
     __shared__ int32_t lds[ROWS * 64];
-    using Stack = WalkStack<64, ROWS>;
-    const Stack S(lds, spill, blockIdx.x * 64 + threadIdx.x, gridDim.x * 64, cap);
+    using Stack = WalkStack<64, ROWS, OWN>;
+    int32_t own[OWN ? OWN : 1];
+    const Stack S(lds, own, spill, blockIdx.x * 64 + threadIdx.x, gridDim.x * 64, cap);
     const uint32_t ray = lane_ray(per_wave, d_count ? min(*d_count, max_count) : max_count);
     float4 p0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), p1 = p0, p2 = p0;
     if (ray != ~0u) {
@@ -134,7 +136,7 @@ __global__ __launch_bounds__(64, 5) void k_world_closest_packed(WorldDev W, cons
                                            hit ? __int_as_float(k.inst) : p2.z, p2.w);
 }
 
-template <int ROWS, bool RESTORE_ALWAYS>
+template <int ROWS, int OWN, bool RESTORE_ALWAYS>
 __global__ __launch_bounds__(64, 5) void k_world_any_packed(WorldDev W, const float4* __restrict__ in,
                                                             uint32_t* __restrict__ out,
                                                             const uint32_t* __restrict__ d_count, uint32_t max_count,
@@ -142,8 +144,9 @@ __global__ __launch_bounds__(64, 5) void k_world_any_packed(WorldDev W, const fl
                                                             int32_t* __restrict__ spill, uint32_t cap,
                                                             uint32_t* __restrict__ ctl, uint32_t per_wave) {
     __shared__ int32_t lds[ROWS * 64];
-    using Stack = WalkStack<64, ROWS>;
-    const Stack S(lds, spill, blockIdx.x * 64 + threadIdx.x, gridDim.x * 64, cap);
+    using Stack = WalkStack<64, ROWS, OWN>;
+    int32_t own[OWN ? OWN : 1];
+    const Stack S(lds, own, spill, blockIdx.x * 64 + threadIdx.x, gridDim.x * 64, cap);
     const uint32_t ray = lane_ray(per_wave, d_count ? min(*d_count, max_count) : max_count);
     float4 p0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), p1 = p0;
     if (ray != ~0u) {
@@ -254,8 +257,8 @@ atlas_rt_status walk_prepare(atlas_rt_world& w, uint32_t count, uint32_t& per_wa
     uint32_t old_cap;
     atlas_rt_status st = world_prepare(w, 0, old_cap);  // the flag block
     cap = w.stack_cap();
-    if (st == ATLAS_RT_OK && cap >= uint32_t(kWalkRows))
-        st = w.spill.ensure(size_t(cap + 1 - kWalkRows) * grid * 64 * sizeof(int32_t));
+    if (const size_t bytes = walk_spill_bytes(cap, kWalkRows + kOwnRows, size_t(grid) * 64); bytes && st == ATLAS_RT_OK)
+        st = w.spill.ensure(bytes);
     return st;
 }
 
@@ -269,7 +272,9 @@ atlas_rt_status launch_world_closest_rays(atlas_rt_world& w, const void* rays, v
     if (st != ATLAS_RT_OK) return st;
     st = w.timing.begin(stream);
     if (st != ATLAS_RT_OK) return st;
-    hipLaunchKernelGGL((k_world_closest_rays<kWalkRows>), dim3(grid), dim3(64), 0, stream, w.dev(),
+    const auto kernel = cap < uint32_t(kWalkRows) ? k_world_closest_rays<kWalkRows, 0>
+                                                  : k_world_closest_rays<kWalkRows, kOwnRows>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, stream, w.dev(),
                        reinterpret_cast<const float4*>(rays), reinterpret_cast<float4*>(hits), inst, count, mask,
                        reinterpret_cast<int32_t*>(w.spill.ptr), cap, reinterpret_cast<uint32_t*>(w.flags.ptr), per_wave);
     ATLAS_HIP_TRY(hipGetLastError());
@@ -282,14 +287,14 @@ atlas_rt_status launch_world_any_rays(atlas_rt_world& w, const void* rays, uint3
     uint32_t per_wave, grid, cap;
     atlas_rt_status st = walk_prepare(w, count, per_wave, grid, cap);
     if (st != ATLAS_RT_OK) return st;
-    if (flags & ATLAS_RT_ANY_RESTORE_ALWAYS)
-        hipLaunchKernelGGL((k_world_any_rays<kWalkRows, true>), dim3(grid), dim3(64), 0, stream, w.dev(),
-                           reinterpret_cast<const float4*>(rays), out, count, mask,
-                           reinterpret_cast<int32_t*>(w.spill.ptr), cap, reinterpret_cast<uint32_t*>(w.flags.ptr), per_wave);
-    else
-        hipLaunchKernelGGL((k_world_any_rays<kWalkRows, false>), dim3(grid), dim3(64), 0, stream,
-                           w.dev(), reinterpret_cast<const float4*>(rays), out, count, mask,
-                           reinterpret_cast<int32_t*>(w.spill.ptr), cap, reinterpret_cast<uint32_t*>(w.flags.ptr), per_wave);
+    const bool restore = (flags & ATLAS_RT_ANY_RESTORE_ALWAYS) != 0;
+    const auto kernel = cap < uint32_t(kWalkRows)
+                            ? (restore ? k_world_any_rays<kWalkRows, 0, true> : k_world_any_rays<kWalkRows, 0, false>)
+                            : (restore ? k_world_any_rays<kWalkRows, kOwnRows, true>
+                                       : k_world_any_rays<kWalkRows, kOwnRows, false>);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, stream, w.dev(), reinterpret_cast<const float4*>(rays), out,
+                       count, mask, reinterpret_cast<int32_t*>(w.spill.ptr), cap,
+                       reinterpret_cast<uint32_t*>(w.flags.ptr), per_wave);
     ATLAS_HIP_TRY(hipGetLastError());
     return ATLAS_RT_OK;
 }
@@ -301,7 +306,9 @@ atlas_rt_status launch_world_closest_packed(atlas_rt_world& w, const void* in, v
     uint32_t per_wave, grid, cap;
     atlas_rt_status st = walk_prepare(w, max_count, per_wave, grid, cap);
     if (st != ATLAS_RT_OK) return st;
-    hipLaunchKernelGGL((k_world_closest_packed<kWalkRows>), dim3(grid), dim3(64), 0, stream, w.dev(),
+    const auto kernel = cap < uint32_t(kWalkRows) ? k_world_closest_packed<kWalkRows, 0>
+                                                  : k_world_closest_packed<kWalkRows, kOwnRows>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, stream, w.dev(),
                        reinterpret_cast<const float4*>(in), reinterpret_cast<float4*>(out), d_count, max_count, tmin,
                        tmax, mask, reinterpret_cast<int32_t*>(w.spill.ptr), cap,
                        reinterpret_cast<uint32_t*>(w.flags.ptr), per_wave);
@@ -350,14 +357,14 @@ atlas_rt_status launch_world_any_packed(atlas_rt_world& w, const void* in, uint3
     uint32_t per_wave, grid, cap;
     atlas_rt_status st = walk_prepare(w, max_count, per_wave, grid, cap);
     if (st != ATLAS_RT_OK) return st;
-    if (flags & ATLAS_RT_ANY_RESTORE_ALWAYS)
-        hipLaunchKernelGGL((k_world_any_packed<kWalkRows, true>), dim3(grid), dim3(64), 0, stream,
-                           w.dev(), reinterpret_cast<const float4*>(in), out, d_count, max_count, tmin, tmax, mask,
-                           reinterpret_cast<int32_t*>(w.spill.ptr), cap, reinterpret_cast<uint32_t*>(w.flags.ptr), per_wave);
-    else
-        hipLaunchKernelGGL((k_world_any_packed<kWalkRows, false>), dim3(grid), dim3(64), 0, stream,
-                           w.dev(), reinterpret_cast<const float4*>(in), out, d_count, max_count, tmin, tmax, mask,
-                           reinterpret_cast<int32_t*>(w.spill.ptr), cap, reinterpret_cast<uint32_t*>(w.flags.ptr), per_wave);
+    const bool restore = (flags & ATLAS_RT_ANY_RESTORE_ALWAYS) != 0;
+    const auto kernel = cap < uint32_t(kWalkRows)
+                            ? (restore ? k_world_any_packed<kWalkRows, 0, true> : k_world_any_packed<kWalkRows, 0, false>)
+                            : (restore ? k_world_any_packed<kWalkRows, kOwnRows, true>
+                                       : k_world_any_packed<kWalkRows, kOwnRows, false>);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, stream, w.dev(), reinterpret_cast<const float4*>(in), out,
+                       d_count, max_count, tmin, tmax, mask, reinterpret_cast<int32_t*>(w.spill.ptr), cap,
+                       reinterpret_cast<uint32_t*>(w.flags.ptr), per_wave);
     ATLAS_HIP_TRY(hipGetLastError());
     return ATLAS_RT_OK;
 }

@@ -123,3 +123,105 @@ def test_launch_shapes_bit_exact(torch_cuda, count, coherent):
     h, s, a = trace(torch_cuda, blas, rays, 0)
     assert np.array_equal(rt_cases.hit_bits(h), rt_cases.hit_bits(ref)) and np.array_equal(s, slots)
     assert np.array_equal(a, oracle_rt.trace_any(nodes, tris, rays))
+
+
+def chain_rays(depth, n):
+    """A tree whose walks hold `depth` stack entries, and n rays that need them all (their tmax ends some early)."""
+    nodes, tris, rays = rt_cases.chain_tree(depth)
+    rays = np.tile(rays, -(-n // len(rays)))[:n]
+    rays["tmax"][1::3] = np.random.default_rng(depth).uniform(90.0, 110.0 + depth, len(rays[1::3])).astype(np.float32)
+    return nodes, tris, rays
+
+
+# the walk's stack rows: 14 in LDS, 32 of the lane's own, then spill rows (30 and 32 for worlds)
+@pytest.mark.parametrize("depth", [12, 13, 14, 15, 28, 29, 30, 31, 44, 45, 46, 47, 60, 61, 62, 63, 80])
+def test_stack_rows_bit_exact(torch_cuda, depth):
+    print("case stack rows", depth, flush=True)
+    torch = torch_cuda
+    nodes, tris, rays = chain_rays(depth, 65536)
+    blas = atlas_rt.Blas.create(nodes, tris)
+    nodes, tris, orig = blas.export()
+    ref, slots = oracle_rt.trace_closest(nodes, tris, orig, rays)
+    any_ref = oracle_rt.trace_any(nodes, tris, rays)
+    assert (slots >= 0).mean() > 0.5
+    for n, kernel in ((65536, 0), (1024, 0), (1024, 1), (65536, 2), (1024, 2 | _abi.KERNEL_LEAF_BATCH)):
+        h, s, a = trace(torch, blas, rays[:n], kernel)
+        assert np.array_equal(rt_cases.hit_bits(h), rt_cases.hit_bits(ref[:n])) and np.array_equal(s, slots[:n]), kernel
+        assert np.array_equal(a, any_ref[:n]), kernel
+    d = torch.from_numpy(rays.view(np.float32).reshape(-1, 8).copy()).cuda()
+    bs = atlas_rt.BatchSet([blas], [(0, 0, len(rays), 0)])
+    for kernel in (1, 2, 2 | _abi.KERNEL_LEAF_BATCH):
+        for block in (64, 256):
+            hits = torch.full((len(rays), 4), -7.0, device="cuda")
+            bs.trace_closest(d, hits, kernel=kernel, block=block, refill=32)
+            h = hits.cpu().numpy().view(atlas_rt.HIT_DTYPE).reshape(-1)
+            assert np.array_equal(rt_cases.hit_bits(h), rt_cases.hit_bits(ref)), (kernel, block)
+    xf = np.zeros((1, 3, 4))
+    xf[0, :, :3] = np.eye(3)
+    w = atlas_rt.World()
+    w.update(atlas_rt.instance_descs(xf, np.zeros(1, np.int64)), [blas])
+    hits = torch.full((len(rays), 4), -7.0, device="cuda")
+    w.trace_closest_rays(d, hits)
+    h = hits.cpu().numpy().view(atlas_rt.HIT_DTYPE).reshape(-1)
+    assert np.array_equal(rt_cases.hit_bits(h), rt_cases.hit_bits(ref))
+
+
+def test_traces_allocate_nothing(torch_cuda):
+    """Once a handle has been traced at all, traces of more rays take no more device memory, so they can be
+    captured; the trees are 19 and more levels deep."""
+    print("case traces without allocation", flush=True)
+    torch = torch_cuda
+    g = W.rng(5, 3)
+    verts = W.triangle_soup(65536, g)
+    rays = W.random_rays(1 << 20, g)
+    d = torch.from_numpy(rays.view(np.float32).reshape(-1, 8).copy()).cuda()
+    hits = torch.empty((len(rays), 4), device="cuda")
+    occluded = torch.empty(len(rays), dtype=torch.int32, device="cuda")
+    xf = np.zeros((1, 3, 4))
+    xf[0, :, :3] = np.eye(3)
+
+    def handles():
+        blas = atlas_rt.Blas.build(verts)
+        assert blas.info()[2] >= 19
+        w = atlas_rt.World()
+        w.update(atlas_rt.instance_descs(xf, np.zeros(1, np.int64)), [blas])
+        few = atlas_rt.BatchSet([blas], [(0, 0, 100, 0)])
+        return blas, w, few, atlas_rt.BatchSet([blas], [(0, 0, len(rays), 0)])
+
+    def traces(blas, w, sets, n):
+        blas.trace_closest(d[:n], hits[:n])
+        blas.trace_any(d[:n], occluded[:n])
+        blas.trace_closest(d[:n], hits[:n], kernel=1)
+        w.trace_closest_rays(d[:n], hits[:n])
+        w.trace_any_rays(d[:n], occluded[:n])
+        sets.trace_closest(d, hits, kernel=1, block=64)
+        sets.trace_closest(d, hits, kernel=2, block=64)
+
+    warm = handles()  # the runtime's own memory for these kernels
+    traces(*warm[:2], warm[3], len(rays))
+    blas, w, few, sets = handles()
+    traces(blas, w, few, 100)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    traces(blas, w, sets, len(rays))
+    torch.cuda.synchronize()
+    assert before - torch.cuda.mem_get_info()[0] < 4 << 20  # of 29 MB that one trace's spill rows would take
+    nodes, tris, orig = blas.export()
+    n = 100000
+    ref, _ = oracle_rt.trace_closest(nodes, tris, orig, rays[:n])
+    # a small trace, then larger ones captured and replayed beside eager work
+    blas2, w2, few2, sets2 = handles()
+    traces(blas2, w2, few2, 100)
+    sets2.trace_closest(d, hits, kernel=2, block=64)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        blas2.trace_closest(d, hits)
+    for rep in range(3):
+        hits.fill_(-3.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        h = hits[:n].cpu().numpy().view(atlas_rt.HIT_DTYPE).reshape(-1)
+        assert np.array_equal(rt_cases.hit_bits(h), rt_cases.hit_bits(ref)), rep
+        blas2.trace_closest(d, hits, kernel=1)
+        blas2.trace_any(d, occluded)
