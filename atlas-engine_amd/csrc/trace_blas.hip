@@ -161,6 +161,9 @@ __global__ __launch_bounds__(BLOCK) void k_blas_closest_persistent(BlasDev B, co
 constexpr uint32_t kChunkWord = 8;  // sequence r's at word kRangeWord * (r + 1) + kChunkWord
 constexpr uint32_t kCoherentWord = 3;
 
+// Chunks of 64 rays in a launch of `count` (not 0) rays, up to 2^32 - 1.
+__device__ __forceinline__ uint32_t chunks_of(uint32_t count) { return (count - 1) / 64u + 1; }
+
 // Whether the wave's rays start and run close together: most lanes within a
 // few degrees of the lane beside them, and within a sixteenth of the tree's
 // box.
@@ -194,7 +197,7 @@ __global__ __launch_bounds__(kBeginBlock) void k_walk_begin(BlasDev B, const flo
     if (tid == 0) coherent = 0;
     __syncthreads();
     constexpr uint32_t kWaves = kBeginBlock / kWave, kEach = 64 / kWaves;
-    const uint32_t chunks = (count + 63u) / 64u;
+    const uint32_t chunks = chunks_of(count);
     uint32_t found = 0;
     for (uint32_t i = 0; i < kEach; i++) {
         const uint32_t k = uint32_t(uint64_t(wave * kEach + i) * chunks / 64u) * 64u + lane;
@@ -260,7 +263,7 @@ __global__ __launch_bounds__(BLOCK, SHAPE == Shape::kPull && ROWS > 14 ? 3 : 5) 
     for (;;) {
         if (kPulls && from >= to && !pull.dry) {
             uint32_t chunk;
-            if (pull.take(ctl + kRangeWord + kChunkWord, kRangeWord, (count + 63u) / 64u, chunk)) {
+            if (pull.take(ctl + kRangeWord + kChunkWord, kRangeWord, chunks_of(count), chunk)) {
                 from = chunk * 64u;
                 to = from + min(64u, count - from);
             }
@@ -394,7 +397,7 @@ constexpr uint32_t kWalkGroups = 5;
 // memory access, and all of its lanes' accesses after one another (5,003 rays
 // 0.111 -> 0.093 ms, 16,384 rays 0.194 -> 0.166 ms against 64 per wave).
 constexpr uint32_t kChooseRays = 65536;
-inline uint32_t rays_per_wave(uint32_t count) { return std::min(64u, (count + 2047u) / 2048u); }
+inline uint32_t rays_per_wave(uint32_t count) { return std::min(64u, (count - 1) / 2048u + 1); }
 
 struct WalkArgs {
     BlasDev B;
@@ -444,9 +447,11 @@ template <bool ANY>
 static atlas_rt_status launch_walk(atlas_rt_blas& blas, const TraceLaunch& L, WalkPlan plan) {
     const uint32_t cap = limit_cap(blas.max_depth + 1, blas.stack_limit);
     // a tree so deep that a wave per 64 rays would need spill rows keeps to the
-    // resident shape, whose lanes are fewer than a large batch's rays
+    // resident shape, whose lanes are fewer than a large batch's rays; so do
+    // more rays than a grid can have threads
     const bool large = plan == WalkPlan::kAuto && L.count >= kChooseRays;
-    const bool choose = large && walk_spill_bytes(cap, kOnceRows<ANY> + kOwnRows, 1) == 0;
+    const bool choose =
+        large && L.count <= UINT32_MAX - 63 && walk_spill_bytes(cap, kOnceRows<ANY> + kOwnRows, 1) == 0;
     const bool pull = large || plan == WalkPlan::kPull || plan == WalkPlan::kPullLeafBatch;
     const bool once = choose || !pull;
     const uint32_t per_wave = once && !choose && plan == WalkPlan::kAuto ? rays_per_wave(L.count) : 64u;

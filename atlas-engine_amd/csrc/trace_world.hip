@@ -249,9 +249,11 @@ static atlas_rt_status world_prepare(atlas_rt_world& w, uint32_t threads, uint32
 namespace {
 
 // Small launches spread over the chip, as those of a single mesh do.
-uint32_t rays_per_wave(uint32_t count) { return std::min(64u, (count + 2047u) / 2048u); }
+uint32_t rays_per_wave(uint32_t count) { return std::min(64u, (count - 1) / 2048u + 1); }
 
 atlas_rt_status walk_prepare(atlas_rt_world& w, uint32_t count, uint32_t& per_wave, uint32_t& grid, uint32_t& cap) {
+    if (count > UINT32_MAX - 63)
+        return fail(ATLAS_RT_E_INVALID_ARG, "world trace: more rays than a launch has threads");
     per_wave = rays_per_wave(count);
     grid = (count - 1) / per_wave + 1;
     uint32_t old_cap;

@@ -218,3 +218,35 @@ def test_gpu_world_packed_ray_interface(torch_cuda):
     ar, _, _ = oracle_rt.trace_world(tl, inst, bl, rr, mask=_abi.MASK_SHADOW, mode=oracle_rt.WORLD_ANY)
     occ = d_occ.cpu().numpy()
     assert np.array_equal(occ[:live], ar["prim_id"][:live]) and np.all(occ[live:] == 0)
+
+
+@pytest.mark.gpu
+def test_gpu_world_packed_count_bound_up_to_the_largest_launch(torch_cuda):
+    """max_count only bounds the device's ray count: any bound up to the most
+    threads of a launch gives the same results, and a larger one is refused."""
+    torch = torch_cuda
+    meshes, descs = small_scene(salt=8, n_inst=5)
+    w, blases = _product_world(meshes, descs)
+    tl, inst, order, bl = _oracle_from_product(w, blases)
+    live = 1000
+    rays = scene_rays(live, 8)
+    packed = np.zeros(live, dtype=atlas_rt.PACKED_RAY_DTYPE)
+    packed["origin"][:, :3] = rays["origin"]
+    packed["origin"][:, 3] = np.arange(live, dtype=np.int32).view(np.float32)
+    packed["direction"][:, :3] = rays["direction"]
+    d_in = torch.from_numpy(packed.view(np.float32).reshape(-1, 12).copy()).cuda()
+    d_count = torch.tensor([live], dtype=torch.int32, device="cuda")
+    rays["tmin"], rays["tmax"] = 0.0, 1e12
+    ref, _, _ = oracle_rt.trace_world(tl, inst, bl, rays, mask=_abi.MASK_SHADOW, mode=oracle_rt.WORLD_ANY)
+    _, slots, _ = oracle_rt.trace_world(tl, inst, bl, rays, mask=_abi.MASK_ALL)
+    for bound in (live, 131072, 131073, 2**32 - 2048, 2**32 - 2047, 2**32 - 64):
+        print("case world packed bound", bound, flush=True)
+        occ = torch.full((live,), -7, dtype=torch.int32, device="cuda")
+        w.trace_any_packed(d_in, occ, d_count, bound)
+        assert np.array_equal(occ.cpu().numpy(), ref["prim_id"])
+        out = torch.zeros_like(d_in)
+        w.trace_closest_packed(d_in, out, d_count, bound)
+        assert np.array_equal(out.view(torch.int32)[:, 9].cpu().numpy(), slots)
+    for bound in (2**32 - 63, 2**32 - 1):
+        with pytest.raises(atlas_rt.AtlasRTError):
+            w.trace_any_packed(d_in, occ, d_count, bound)
