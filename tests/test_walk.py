@@ -107,6 +107,94 @@ def test_hard_rays_bit_exact(torch_cuda, name):
     assert len(bad) == 0, f"{name} any: {len(bad)} rays, first {bad[:4]} {rays[bad[:2]]}"
 
 
+def test_hard_rays_batched_bit_exact(torch_cuda):
+    torch = torch_cuda
+    g = W.rng(5, 4)
+    M = list(meshes(g).values())
+    blases = [atlas_rt.Blas.build(v) for v in M]
+    n = 20011
+    rays = np.concatenate([hard_rays(g, v, n) for v in M])
+    rays["direction"][::97] = np.nan
+    bs = atlas_rt.BatchSet(blases, [(k, k * n, n, 0) for k in range(len(M))])
+    ref = np.zeros(len(rays), atlas_rt.HIT_DTYPE)
+    for k, b in enumerate(blases):
+        ref[k * n:(k + 1) * n] = oracle_rt.trace_closest(*b.export(), rays[k * n:(k + 1) * n])[0]
+    d = torch.from_numpy(rays.view(np.float32).reshape(-1, 8).copy()).cuda()
+    for kernel in (1, 2, 2 | _abi.KERNEL_LEAF_BATCH):
+        for block in (64, 128, 256):
+            print("case hard rays batched", kernel, block, flush=True)
+            h = torch.full((len(rays), 4), -7.0, device="cuda")
+            bs.trace_closest(d, h, kernel=kernel, block=block, refill=32)
+            h = h.cpu().numpy().view(atlas_rt.HIT_DTYPE).reshape(-1)
+            bad = np.nonzero(np.any(rt_cases.hit_bits(h) != rt_cases.hit_bits(ref), axis=1))[0]
+            assert len(bad) == 0, f"{kernel} {block}: {len(bad)} rays, first {bad[:4]} {rays[bad[:2]]} {h[bad[:2]]} {ref[bad[:2]]}"
+
+
+def transforms(g, size):
+    """Instance matrices: as they are, turned by a quarter (components that become exactly 0), any rotation, mirrored
+    and scaled unevenly, flat, tiny (object-space directions of 1e30) and as large as finite boxes of a mesh of this
+    size allow (directions of 1e-35 and less, subnormal components among them)."""
+    quarter = np.array([[0, 0, 1.0], [0, 1, 0], [-1, 0, 0]])
+    c, s = np.cos(0.7), np.sin(0.7)
+    turn = np.array([[c, -s, 0], [s, c, 0], [0, 0, 1.0]])
+    linear = [np.eye(3), quarter, turn, np.diag([-1.0, 2.0, 0.25]), turn @ np.diag([1.0, 1e-3, 1.0]), np.eye(3) * 1e-30,
+              quarter * (1e36 / size), np.eye(3), turn @ quarter]
+    m = np.zeros((len(linear), 3, 4))
+    for k, a in enumerate(linear):
+        m[k, :, :3] = a
+        m[k, :, 3] = np.round(g.uniform(-6, 6, 3) * 2) / 2 if k else 0.0
+    return m
+
+
+@pytest.mark.parametrize("name", ["soup", "boxes", "height", "strip", "one", "chain"])
+def test_hard_rays_through_worlds_bit_exact(torch_cuda, name):
+    """Overlapping instances, so that walks leave instances with TLAS entries on the stack; some masked from one of
+    the two masks.  The chain's walks hold 80 entries above the TLAS's."""
+    torch = torch_cuda
+    g = W.rng(5, 5)
+    if name == "chain":
+        nodes, tris, _ = rt_cases.chain_tree(80)
+        first = atlas_rt.Blas.create(nodes, tris)
+        verts = np.concatenate([tris["v0"][:, :3], tris["v1"][:, :3], tris["v2"][:, :3]], axis=1)
+    else:
+        verts = meshes(g)[name]
+        first = atlas_rt.Blas.build(verts)
+    second = atlas_rt.Blas.build(boxes_mesh(g, 40))
+    xf = transforms(g, np.abs(verts).max())
+    xf = np.concatenate([xf, xf[:4]])
+    xf[-4:, :, 3] += 0.5
+    descs = atlas_rt.instance_descs(xf, [0] * 9 + [1] * 4)
+    descs["mask"][[2, 7, 10]] = _abi.MASK_ALL
+    descs["mask"][[3, 11]] = _abi.MASK_SHADOW
+    w = atlas_rt.World()
+    w.update(descs, [first, second])
+    tl, inst, order = w.export()
+    bl = [first.export(), second.export()]
+    rays = hard_rays(g, verts, 30011)
+    if name == "chain":
+        rays[::2] = np.resize(rt_cases.chain_tree(80)[2], len(rays[::2]))
+    rays["direction"][::97] = np.nan
+    d = torch.from_numpy(rays.view(np.float32).reshape(-1, 8).copy()).cuda()
+    for mask in (_abi.MASK_ALL, _abi.MASK_SHADOW):
+        print("case hard rays world", name, mask, flush=True)
+        h = torch.full((len(rays), 4), -7.0, device="cuda")
+        gi = torch.full((len(rays),), -7, dtype=torch.int32, device="cuda")
+        w.trace_closest_rays(d, h, gi, mask=mask)
+        h = h.cpu().numpy().view(atlas_rt.HIT_DTYPE).reshape(-1)
+        ref, _, ri = oracle_rt.trace_world(tl, inst, bl, rays, mask=mask)
+        ri = np.where(ri >= 0, order[np.maximum(ri, 0)].astype(np.int32), -1)
+        bad = np.nonzero(np.any(rt_cases.hit_bits(h) != rt_cases.hit_bits(ref), axis=1) | (gi.cpu().numpy() != ri))[0]
+        assert len(bad) == 0, f"{len(bad)} rays, first {bad[:4]} {rays[bad[:2]]} {h[bad[:2]]} {ref[bad[:2]]}"
+        assert (ri >= 0).sum() > 1000
+        for flags, mode in ((_abi.ANY_ENGINE_HITANY, oracle_rt.WORLD_ANY),
+                            (_abi.ANY_RESTORE_ALWAYS, oracle_rt.WORLD_ANY_RESTORE)):
+            a = torch.full((len(rays),), -7, dtype=torch.int32, device="cuda")
+            w.trace_any_rays(d, a, mask=mask, flags=flags)
+            ar, _, _ = oracle_rt.trace_world(tl, inst, bl, rays, mask=mask, mode=mode)
+            bad = np.nonzero(a.cpu().numpy() != ar["prim_id"])[0]
+            assert len(bad) == 0, f"any {flags}: {len(bad)} rays, first {bad[:4]} {rays[bad[:2]]}"
+
+
 @pytest.mark.parametrize("count", [1, 2, 63, 64, 65, 2048, 2049, 5003, 65535, 65536, 65537, 131073])
 @pytest.mark.parametrize("coherent", [False, True])
 def test_launch_shapes_bit_exact(torch_cuda, count, coherent):
