@@ -62,6 +62,38 @@ def test_resident_equals_wavefront_opaque(torch_cuda, fif):
     assert len(diff[0]) == 0, f"{len(diff[0])} pixels differ, first {list(zip(*diff))[:5]}"
 
 
+def test_resident_equals_wavefront_axis_aligned(torch_cuda):
+    """Boxes on a lattice, as they are and turned by a quarter, seen along an axis from a lattice point: flat and
+    shared box planes and rays with zero components, which the resident kernel's walk settles in its later stages and
+    the bounce-by-bounce kernels by the engine's arithmetic alone."""
+    print("case resident axis aligned", flush=True)
+    g = W.rng(2, 701)
+    lo = g.integers(-8, 8, (300, 3)) * 0.5
+    hi = lo + g.integers(1, 4, (300, 3)) * 0.5
+    at = np.stack([np.where((np.arange(8) >> k) & 1, hi[:, k:k + 1], lo[:, k:k + 1]) for k in range(3)], axis=-1)
+    faces = [(0, 2, 3, 1), (4, 5, 7, 6), (0, 1, 5, 4), (2, 6, 7, 3), (0, 4, 6, 2), (1, 3, 7, 5)]
+    verts = np.concatenate([at[:, [f[0], f[1], f[2], f[0], f[2], f[3]]].reshape(-1, 9) for f in faces]).astype(np.float32)
+    t = verts.reshape(-1, 3, 3).astype(np.float64)
+    normal = np.cross(t[:, 0] - t[:, 1], t[:, 0] - t[:, 2])
+    normal /= np.linalg.norm(normal, axis=1, keepdims=True)
+    blas = atlas_rt.Blas.build(verts)
+    blas.set_shading(np.tile(normal, (1, 3)).astype(np.float32))
+    xf = np.zeros((3, 3, 4))
+    xf[:, :, :3] = [np.eye(3), [[0, 0, 1], [0, 1, 0], [-1, 0, 0]], [[0, -1, 0], [1, 0, 0], [0, 0, 1]]]
+    xf[:, :, 3] = [[0, 0, 0], [0.5, 0, 1], [-1, 0.5, 0]]
+    w_ = atlas_rt.World()
+    w_.update(atlas_rt.instance_descs(xf, np.zeros(3, np.int64)), [blas])
+    mats = W.c2_materials({"albedo": np.full((1, 3), 0.6, np.float32), "roughness": np.ones(1, np.float32)})
+    W_, H_ = 97, 65
+    for yaw in (0.0, 90.0):
+        cam = atlas_rt.camera((0.5, 0.5, -16.0) if yaw == 0.0 else (-16.0, 0.5, 0.5), yaw, 0.0, 50.0, W_ / H_)
+        a, b = _both(lambda wf: atlas_rt.PathTracer(w_, W_, H_, 4, mats, W.sun_light(), env=ENV, wavefront=wf),
+                     lambda pt: pt.render(cam, 5), lambda pt: pt.read().cpu().numpy())
+        assert np.all(a[..., 3] == 5) and len(np.unique(a[..., 0])) > 100
+        diff = np.nonzero(np.any(a.view(np.uint32) != b.view(np.uint32), axis=-1))
+        assert len(diff[0]) == 0, f"{len(diff[0])} pixels differ, first {list(zip(*diff))[:5]}"
+
+
 def test_resident_batches_equal_wavefront(torch_cuda):
     """19 frames in one call run as resident launches of 8, 8 and 3 frames
     (each frame its own seeds and radiance buffer, summed per pixel in frame

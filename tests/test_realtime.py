@@ -205,12 +205,36 @@ def test_gpu_realtime_matches_oracle(torch_cuda, spf):
     pt.close()
 
 
+def _uniform(img, x0, x1, y0, y1):
+    """Whether the image has one value over [x0, x1) x [y0, y1), clamped to it."""
+    cut = img[max(y0, 0):y1, max(x0, 0):x1]
+    return bool((cut == cut[:1, :1]).all())
+
+
+def _check_flat_equals_taps(depth, frame, res):
+    """Without a history the resolve is the neighbourhood's mean: that of a pixel in a tile of one value (16 x 16 and
+    5 around) is that of a pixel in a mixed tile, which takes the taps, where both read the same values (5 around)."""
+    H_, W_ = depth.shape
+    img = np.concatenate([frame[..., :3], depth[..., None]], axis=-1)
+    kinds = {True: [], False: []}
+    for y in range(H_):
+        for x in range(W_):
+            if _uniform(img, x - 5, x + 6, y - 5, y + 6):
+                tx, ty = x // 16 * 16, y // 16 * 16
+                kinds[_uniform(img, tx - 5, tx + 21, ty - 5, ty + 21)].append((y, x))
+    assert len(kinds[True]) > 50 and len(kinds[False]) > 50
+    pix = np.array(kinds[True] + kinds[False])
+    values = np.concatenate([img[pix[:, 0], pix[:, 1]], res[pix[:, 0], pix[:, 1]]], axis=1).view(np.uint32)
+    assert len(np.unique(values, axis=0)) == 1
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("yaw", [0.0, 35.0, 180.0])
 def test_gpu_resolve_of_flat_tiles(torch_cuda, yaw):
     """Tiles of one texel value sum it without taps, and unmoved history texels
     skip the normal and depth agreement: the scene ahead, half of it and only
-    sky, at a ragged size, two frames from one place."""
+    sky, at a ragged size, two frames from one place.  Where half of the
+    picture is sky, the flat tiles' sums are those of the taps bit for bit."""
     print(f"case resolve flat tiles yaw={yaw}", flush=True)
     S = _scene()
     W_, H_ = 83, 61
@@ -233,8 +257,10 @@ def test_gpu_resolve_of_flat_tiles(torch_cuda, yaw):
         # the taps' hardware exp2 and division: the bound of the test above
         assert (np.abs(res - ref) <= 1e-6 + 1e-5 * np.abs(ref)).all(axis=-1).mean() > 0.999
         hist = dict(hdepth=depth, hnormal=nrm, hmaterial=mat, hradiance=res)
+        if yaw == 35.0 and f == 0:
+            _check_flat_equals_taps(depth, got[_abi.RT_FRAME], res)
     if yaw == 180.0:
-        assert len(np.unique(got[_abi.RT_FRAME][..., :3].reshape(-1, 3), axis=0)) == 1
+        assert len(np.unique(depth)) == 1 and len(np.unique(got[_abi.RT_FRAME][..., :3].reshape(-1, 3), axis=0)) == 1
     pt.close()
 
 
