@@ -399,6 +399,16 @@ constexpr uint32_t kWalkGroups = 5;
 constexpr uint32_t kChooseRays = 65536;
 inline uint32_t rays_per_wave(uint32_t count) { return std::min(64u, (count - 1) / 2048u + 1); }
 
+// Whether any-hit rays may be worth refilling.  Their walks are short, and the
+// shorter the smaller the tree, so that refills cost more than the idle lanes
+// do until there are many rays.  Incoherent rays, refilled / once, us: 1,500
+// triangles 91 / 43 at 131,072 rays, 575 / 591 at 4 M; 5,000: 330 / 283 at 1 M,
+// 481 / 526 at 2 M; 20,011: 270 / 177 at 300,000, 330 / 320 at 600,000, 434 /
+// 502 at 1 M; 65,536: 347 / 297 at 300,000, 441 / 523 at 600,000.
+inline bool pays_any(uint32_t count, uint32_t nodes) {
+    return uint64_t(count) * std::min(nodes, 16384u) >= uint64_t(1) << 33;
+}
+
 struct WalkArgs {
     BlasDev B;
     const float4* rays;
@@ -449,9 +459,10 @@ static atlas_rt_status launch_walk(atlas_rt_blas& blas, const TraceLaunch& L, Wa
     // a tree so deep that a wave per 64 rays would need spill rows keeps to the
     // resident shape, whose lanes are fewer than a large batch's rays; so do
     // more rays than a grid can have threads
-    const bool large = plan == WalkPlan::kAuto && L.count >= kChooseRays;
-    const bool choose =
-        large && L.count <= UINT32_MAX - 63 && walk_spill_bytes(cap, kOnceRows<ANY> + kOwnRows, 1) == 0;
+    const bool deep = walk_spill_bytes(cap, kOnceRows<ANY> + kOwnRows, 1) != 0;
+    const bool large = plan == WalkPlan::kAuto && L.count >= kChooseRays &&
+                       (!ANY || deep || pays_any(L.count, uint32_t(blas.nodes.size())));
+    const bool choose = large && L.count <= UINT32_MAX - 63 && !deep;
     const bool pull = large || plan == WalkPlan::kPull || plan == WalkPlan::kPullLeafBatch;
     const bool once = choose || !pull;
     const uint32_t per_wave = once && !choose && plan == WalkPlan::kAuto ? rays_per_wave(L.count) : 64u;

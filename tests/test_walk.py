@@ -213,6 +213,27 @@ def test_launch_shapes_bit_exact(torch_cuda, count, coherent):
     assert np.array_equal(a, oracle_rt.trace_any(nodes, tris, rays))
 
 
+@pytest.mark.parametrize("more", [-1, 0, 4097])
+@pytest.mark.parametrize("coherent", [False, True])
+def test_any_hit_shapes_bit_exact(torch_cuda, more, coherent):
+    """Any-hit rays are refilled, if incoherent, from 2^33 / nodes of them on."""
+    print("case any-hit shapes", more, coherent, flush=True)
+    torch = torch_cuda
+    blas = atlas_rt.Blas.build(W.heightfield(129))
+    nodes, tris, orig = blas.export()
+    count = -(-2**33 // min(len(nodes), 16384)) + more
+    if coherent:
+        rays = W.pinhole_rays(1024, 517, (64.0, 60.0, -19.0), 0.0, 30.0)[:count]
+    else:
+        rays = W.random_rays(count, W.rng(5, 6), extent=80.0)
+    assert len(rays) == count
+    d = torch.from_numpy(rays.view(np.float32).reshape(-1, 8).copy()).cuda()
+    a = torch.full((count,), -7, dtype=torch.int32, device="cuda")
+    blas.trace_any(d, a)
+    ref = oracle_rt.trace_any(nodes, tris, rays)
+    assert ref.mean() > 0.05 and np.array_equal(a.cpu().numpy().astype(np.uint32), ref)
+
+
 def chain_rays(depth, n):
     """A tree whose walks hold `depth` stack entries, and n rays that need them all (their tmax ends some early)."""
     nodes, tris, rays = rt_cases.chain_tree(depth)
