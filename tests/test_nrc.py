@@ -235,6 +235,21 @@ def test_gpu_nrc_infer_is_the_same_at_every_batch_size(torch_cuda, tiles):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 15, 16, 17])
+def test_gpu_nrc_infer_of_few_queries(torch_cuda, n):
+    """Up to 16 queries are gathered by four lanes each: the same bits as in a larger batch."""
+    print("case nrc infer few", n, flush=True)
+    torch = torch_cuda
+    g = np.random.default_rng(16)
+    rc = _cache(torch)
+    _set_random(torch, rc, g, _oracle_params())
+    q = torch.from_numpy(rand_queries(g, 256)).cuda()
+    out = torch.full((n + 3, 4), -7.0, device="cuda")
+    rc.infer(q[:n].contiguous(), out)
+    assert torch.equal(out[:n], rc.infer(q)[:n]) and bool((out[n:] == -7.0).all())
+
+
+@pytest.mark.gpu
 def test_gpu_nrc_gradients_match_oracle(torch_cuda):
     print("case nrc gradients", flush=True)
     torch = torch_cuda
