@@ -386,10 +386,12 @@ static atlas_rt_status ensure_flags(atlas_rt_blas& blas) {
 constexpr int kWalkBlock = 256;
 // LDS stack rows: with the staged nodes, five groups of resident waves fit
 // one CU (14 KB + 16.3 KB each); of the waves that run once, as many as the
-// registers allow (20 of 7.7 KB each, for any hit 28 of 5.6 KB).
+// registers allow, 20 and, for any hit, 28 (LDS is allocated in pieces of
+// 1,280 B: 7,680 and 5,120 B per wave; with 22 rows only 25 waves fit, and
+// 877,536 shadow rays over 2.1M triangles take 125 us, not 118).
 constexpr int kWalkRows = 14;
 template <bool ANY>
-constexpr int kOnceRows = ANY ? 22 : 30;
+constexpr int kOnceRows = ANY ? 20 : 30;
 constexpr uint32_t kWalkGroups = 5;
 
 // Launches below this many rays run once, with as many rays per wave as give

@@ -242,8 +242,8 @@ def chain_rays(depth, n):
     return nodes, tris, rays
 
 
-# the walk's stack rows: 14 in LDS, 32 of the lane's own, then spill rows (30 and 32 for worlds)
-@pytest.mark.parametrize("depth", [12, 13, 14, 15, 28, 29, 30, 31, 44, 45, 46, 47, 60, 61, 62, 63, 80])
+# the walk's stack rows: 14 in LDS (20 or 30 with a wave per ray set and in worlds), 32 of the lane's own, then spill rows
+@pytest.mark.parametrize("depth", [12, 13, 14, 15, 18, 19, 20, 28, 29, 30, 31, 44, 45, 46, 47, 50, 51, 52, 60, 61, 62, 63, 80])
 def test_stack_rows_bit_exact(torch_cuda, depth):
     print("case stack rows", depth, flush=True)
     torch = torch_cuda
