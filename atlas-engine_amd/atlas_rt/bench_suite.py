@@ -444,11 +444,13 @@ def _study(torch, log, name, meshes, mats, xf, which, cc, bounds, ref_spp, bounc
     width, height = cc["width"], cc["height"]
     cam = camera(cc["eye"], cc["yaw_deg"], cc["pitch_deg"], cc["fov_y_deg"], width / height)
     ref_pt = PathTracer(w, width, height, bounces, mats, sun, env=W.C2_ENV)
+    short = name.split(":")[0]
     t_ref = 0.0
     chunk = 256
     for k in range(0, ref_spp, chunk):
         t_ref += _sync_time(torch, lambda: ref_pt.render(cam, min(chunk, ref_spp - k)))
-        log(f"{name}: reference {k + chunk} / {ref_spp} spp")
+        if (k // chunk) % 4 == 3:
+            log(f"{short}: reference {k + chunk} / {ref_spp} spp")
     ref = ref_pt.read().clone()
     del ref_pt
     plain = _curve(torch, PathTracer(w, width, height, bounces, mats, sun, env=W.C2_ENV), cam, ref, checkpoints)
@@ -468,7 +470,8 @@ def _study(torch, log, name, meshes, mats, xf, which, cc, bounds, ref_spp, bounc
                 continue
             t_c = _time_to(cache, e_p)
             speedups[str(spp)] = None if t_c is None else round(t_p / t_c, 3)
-        log(f"{name}: stride {train_stride} steps {train_steps} warm-up {warmup} lag {lag}: speedups {speedups}")
+        log(f"{short}: stride {train_stride} steps {train_steps} warm-up {warmup} lag {lag}: speedups at 16 / 64 / 256 "
+            f"spp {speedups.get('16')} / {speedups.get('64')} / {speedups.get('256')}")
         runs.append({
             "train_stride": train_stride, "train_steps_per_frame": train_steps, "warmup_frames": warmup,
             "query_lag": lag,

@@ -65,9 +65,28 @@ def parse():
     ap.add_argument("--cpu-seconds", type=float, default=15.0, help="target CPU work for the baseline sample")
     ap.add_argument("--no-extra", action="store_true", help="only the c0 headline (skip c1, c3 and the cache study)")
     ap.add_argument("--ref-spp", type=int, default=4096, help="samples per pixel of the plain reference render")
+    ap.add_argument("--details", metavar="FILE", help="write every field there too: the printed line leaves out the "
+                                                      "autotuner's trials and the cache study's curves")
     ap.add_argument("--probe", nargs="+", metavar="ARG",
                     help="run one fixed profiler workload instead of the benchmark (see PROBES)")
     return ap.parse_args()
+
+
+def headline(out):
+    """The record without its long lists, so that the line stays under 12 KB."""
+    out = json.loads(json.dumps(out))
+    if "c3" in out:
+        out["c3"]["trials"] = len(out["c3"]["trials"])
+    for k in ("dense", "c2_layout"):
+        study = out.get("radiance_cache", {}).get(k)
+        if study:
+            del study["plain_curve"]
+            study["runs"] = [{"stride": r["train_stride"], "steps": r["train_steps_per_frame"],
+                              "warmup": r["warmup_frames"], "lag": r["query_lag"],
+                              "speedup": [r["speedup_to_plain_rel_mse_at_spp"].get(n) for n in ("16", "64", "256")]}
+                             for r in study.pop("cache_runs")]
+            study["runs_note"] = "speedup at the plain tracer's rel-MSE after 16, 64 and 256 spp"
+    return out
 
 
 def log(msg):
@@ -78,7 +97,7 @@ def log(msg):
 # traffic it reports belongs to that kernel only.
 PMC_SUMMARIES = {18: os.path.join(ROOT, "profiles", "k_blas_closest_persistent_regstack_c0_pmc.md"),
                  50: os.path.join(ROOT, "profiles", "k_blas_closest_persistent_regstack_fslab_c0_pmc.md"),
-                 66: os.path.join(ROOT, "profiles", "k_blas_closest_persistent_leafbatch_c0_pmc.md")}
+                 66: os.path.join(ROOT, "profiles", "k_blas_walk_c0_pmc.md")}
 
 
 def pmc_traffic(kernel):
@@ -501,7 +520,7 @@ def probe_c3(kernel=66, block=256, refill=32, reps=4):
     print(f"c3 probe done: {len(rays)} rays, kernel {kernel} block {block}", flush=True)
 
 
-def summarize_pmc(out_dir, kernel_re=r"k_blas_closest|k_batch"):
+def summarize_pmc(out_dir, kernel_re=r"k_blas_closest|k_blas_walk|k_batch"):
     """Per-dispatch counter averages of the copy and the trace kernels, and
     the trace kernel's traffic scaled by the copy's known bytes."""
     import csv
@@ -726,11 +745,14 @@ def main():
         out["c3"] = bench_suite.c3(torch, log)
         if not args.no_cpu_baseline:
             out["cpu_configs"] = cpu_configs(out, host_cpu()["threads"])
-            log(f"cpu configs: {json.dumps(out['cpu_configs'])}")
+            log("cpu configs done")
         for k in ("c1", "c2", "c3"):
             out[k].pop("_check", None)
         out["radiance_cache"] = bench_suite.cache_study(torch, log, args.ref_spp)
-    print(json.dumps(out), flush=True)
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(out, f, indent=1)
+    print(json.dumps(headline(out)), flush=True)
 
 
 if __name__ == "__main__":
