@@ -452,8 +452,8 @@ __global__ __launch_bounds__(64, 2) void k_nrc_infer(NrcDev P, const float4* __r
 // The activations that the backward pass needs, its accumulators and the
 // wave's tiles of the weight gradient fill the registers of one wave per SIMD
 // (at 256, two waves, they spill: a training step of 65,536 queries takes
-// 344 us and not 327).  The scatter into the table is the largest part, about
-// 200 us.  Adding each step's weight gradient into LDS with atomics took a
+// 344 us and not 327).  The scatter into the table is the largest part, 175 of
+// the kernel's 256 us.  Adding each step's weight gradient into LDS with atomics took a
 // third of the kernel: the step 486 -> 327 us, 1,024 queries 159 -> 69,
 // 300,000 queries 1,950 -> 1,150.
 __global__ __launch_bounds__(kTrainBlock, 1) void k_nrc_train(NrcDev P, const float4* __restrict__ q,
@@ -621,7 +621,7 @@ __device__ __forceinline__ void put_weight(uint32_t j, uint16_t w, uint16_t* wn,
 // Sums the blocks' weight gradients, 64 weights per group: wave w of four adds
 // every fourth block's (coalesced, eight loads in flight), then the first
 // adds the four sums.  One thread per weight instead walks all the blocks on
-// a quarter of the chip (256 blocks: 62 us against 9).
+// a quarter of the chip (256 blocks: 62 us against 6).
 constexpr uint32_t kReduceWeights = 64, kReduceWaves = 4;
 __global__ __launch_bounds__(kReduceWeights * kReduceWaves) void k_mlp_reduce(
     const float* __restrict__ partial, uint32_t blocks, float* __restrict__ grad_out, float* __restrict__ master,

@@ -735,11 +735,11 @@ __global__ __launch_bounds__(BLOCK) void k_shadow(WorldDev W, const FrameCtl* __
 // launch waits for the slowest path of a bounce before the next bounce
 // starts: the frame's only tail is its slowest whole path.  Lanes that trace
 // closest hits and lanes that trace shadow rays share one step body over
-// opaque worlds (world_walk).  Shading is batched per wave: the wave
-// keeps stepping until its busy lanes have all finished a walk (kShadeDiv
-// = 1; 1 / kShadeDiv of them in general), then those lanes shade or add
-// their shadow ray's light together.  Paths refill idle lanes between
-// batches (one atomic per wave).
+// opaque worlds (world_walk).  Shading is batched per wave: the wave keeps
+// stepping until all of its busy lanes have finished a walk (over worlds with
+// opacity 1 / kShadeDiv of them), then those lanes shade or add their shadow
+// ray's light together.  Paths refill idle lanes between batches (one atomic
+// per wave).
 //
 // Every path runs the same arithmetic in the same order as in the
 // bounce-by-bounce kernels (raygen, k_trace, shade_path, k_shadow), and

@@ -3,9 +3,10 @@
 // Work item w in [0, total) belongs to the batch b with prefix[b] <= w <
 // prefix[b+1] (binary search over the exclusive prefix of the batch sizes);
 // its ray is rays[batch[b].ray_offset + (w - prefix[b])] and it is traced
-// against blases[batch[b].blas] with one of the step functions of
-// trace_core.h: binary nodes in engine order, or 4- / 8-wide nodes, each
-// with the stack in LDS or with its top in registers.
+// against blases[batch[b].blas]: binary nodes in engine order on the filtered
+// walk of walk.h (k_batch_walk), or the autotuner's other candidates with the
+// step functions of trace_core.h (k_batch_persistent, k_batch_grid): the stack's
+// top in registers, the widened float slab test, 4- / 8-wide nodes.
 //
 // Launch shapes (picked by the autotuner):
 //  * persistent<BLOCK>: resident waves pull work items from a global counter

@@ -222,11 +222,11 @@ __global__ __launch_bounds__(kBeginBlock) void k_walk_begin(BlasDev B, const flo
 // (kPull); a large batch launches both.  Coherent rays share their nodes'
 // cache lines and end together: a wave per chunk, started in the rays' order
 // by the hardware, loads each node once for many lanes and balances best
-// (1920 x 1080 camera rays over 1.0M triangles: 0.26 ms against 0.39
-// resident).  Incoherent rays end one by one, so lanes are refilled, and their
+// (kernel time of 1920 x 1080 camera rays over 1.0M triangles: 0.26 ms against
+// 0.39 resident).  Incoherent rays end one by one, so lanes are refilled, and their
 // node records go through LDS (NodeStage) while there is work; the last rays,
 // few in each wave, load their nodes directly (1M rays in a random soup of
-// 65,536 triangles: 0.60 ms against 0.84 once).
+// 65,536 triangles: 0.62 ms against 0.90 once).
 //
 // When to refill.  A wave waits until its idle lanes have cost kIdleSteps
 // lane-steps since its last refill, about what a refill costs.  The rays of a

@@ -198,10 +198,14 @@ atlas_rt_status atlas_rt_blas_export(const atlas_rt_blas* blas, atlas_rt_gpu_bvh
 /* Bulk tracing against one BLAS                                             */
 /* ------------------------------------------------------------------------- */
 
-/* Traversal kernels.  ATLAS_RT_KERNEL_AUTO picks the default (single BLAS:
- * leaf-batched resident waves, BVH2_PERSISTENT | LEAF_BATCH, from 65,536 rays
- * up; one ray per lane, BVH2_EXACT, below) or the autotuned variant (batch
- * sets).
+/* Traversal kernels.  ATLAS_RT_KERNEL_AUTO picks the default or, for batch
+ * sets, the autotuned variant.  Single BLAS: below 65,536 rays one ray per
+ * lane, spread over the chip; from there on the rays are sampled on the
+ * device, coherent ones run one ray per lane (BVH2_EXACT), others on
+ * leaf-batched resident waves (BVH2_PERSISTENT | LEAF_BATCH).  Any-hit traces
+ * run one ray per lane up to 2^33 / nodes rays (524,288 from 16,384 nodes up)
+ * and choose as above from there on, whatever kernel is named.  All of these
+ * give the same results bit for bit.
  *  BVH2_EXACT       one ray per lane over the engine's binary nodes, engine order
  *  BVH2_PERSISTENT  resident waves refilled with new rays, same traversal
  *  BVH4 / BVH8      resident waves over 4- / 8-wide nodes collapsed from the
@@ -242,7 +246,13 @@ atlas_rt_status atlas_rt_blas_export(const atlas_rt_blas* blas, atlas_rt_gpu_bvh
  * wave counters, traversal stack spill and overflow flag in the BLAS, so they
  * are stream-ordered: traces of the same BLAS on different streams must not
  * overlap (make one stream wait on an event recorded after the other's
- * trace).  Traces of different BLASes are independent. */
+ * trace).  Traces of different BLASes are independent.
+ * Memory: the first trace of a BLAS allocates its flags (1.2 KB).  AUTO,
+ * BVH2_EXACT, BVH2_PERSISTENT and any-hit traces of trees of up to 44 levels
+ * allocate nothing else, whatever their ray count.  For deeper trees, and with
+ * the other kernel bits, the first trace that needs stack spill rows allocates
+ * them and one that needs more replaces them: a graph that holds such a trace
+ * must not be launched after a larger trace. */
 atlas_rt_status atlas_rt_trace_closest_rays(const atlas_rt_blas* blas, const atlas_rt_ray* d_rays,
                                             atlas_rt_hit* d_hits, int32_t* d_slot, uint32_t count,
                                             int32_t kernel, void* stream);
