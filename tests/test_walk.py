@@ -275,6 +275,27 @@ def test_stack_rows_bit_exact(torch_cuda, depth):
     assert np.array_equal(rt_cases.hit_bits(h), rt_cases.hit_bits(ref))
 
 
+@pytest.mark.parametrize("limit", [1, 2, 12, 13, 14, 18, 19, 20, 21, 28, 29, 30, 31, 44, 45, 46, 47, 50, 51, 52])
+def test_stack_limits_at_the_rows_edges(torch_cuda, limit):
+    """A walk of a chain of d levels holds d entries: a limit of d is enough for it and one of d - 1 stops every ray,
+    on each side of the rows' edges, in every shape."""
+    print("case stack limit", limit, flush=True)
+    torch = torch_cuda
+    for depth in (limit, limit + 1):
+        nodes, tris, rays = rt_cases.chain_tree(depth)
+        rays = np.tile(rays, 64)
+        blas = atlas_rt.Blas.create(nodes, tris)
+        blas.set_stack_limit(limit)
+        for n, kernel in ((len(rays), 0), (1024, 0), (1024, 1), (1024, 2), (1024, 2 | _abi.KERNEL_LEAF_BATCH)):
+            h, s, a = trace(torch, blas, rays[:n], kernel)
+            assert blas.trace_status() == (_abi.OK if depth == limit else _abi.E_STACK_OVERFLOW), (depth, kernel)
+            if depth == limit:
+                assert np.all(h["prim_id"] >= 0) and np.all(s >= 0) and np.all(a == 1), (depth, kernel)
+            else:
+                assert np.all(h["prim_id"] == -1) and np.all(s == -1) and np.all(a == 0), (depth, kernel)
+                assert np.array_equal(h["t"], rays["tmax"][:n])
+
+
 def test_traces_allocate_nothing(torch_cuda):
     """Once a handle has been traced at all, traces of more rays take no more device memory, so they can be
     captured; the trees are 19 and more levels deep."""
